@@ -45,3 +45,19 @@ def test_factory_rejects_unknown_types_without_gpu():
                  (b"3D", b"viscoelastic"), (b"2D", b"viscotmem"), (b"2D", b"viscoemem")):
         assert lib.wv_create(d, t, ctypes.byref(h)) == 0, (d, t)
         lib.wv_destroy(h)
+
+
+def test_depth_parts_are_never_empty():
+    """The 3D kernels' parts along depth (wv::depth_parts): every part holds planes, and the rule's
+    bounds (at least max(4H, 8) planes wanted per part, no more parts than the block count asks for) hold."""
+    f = ctypes.CDLL(abi.LIB_PATH)["_ZN2wv11depth_partsEiiii"]
+    f.argtypes, f.restype = [ctypes.c_int] * 4, ctypes.c_int
+    for H in range(1, 7):
+        for tiles in (1, 7, 96, 480, 1500, 20000):
+            for NY in range(2, 420):
+                n = f(NY, H, tiles, 12288)
+                wanted = max(1, min(-(-12288 // tiles), NY // max(4 * H, 8)))
+                assert 1 <= n <= wanted
+                planes = -(-NY // n)
+                assert (n - 1) * planes < NY <= n * planes, (NY, H, tiles, n)
+                assert planes == -(-NY // wanted)

@@ -94,3 +94,8 @@ def test_acoustic3d_batched_equals_single_and_graphs():
         single = cases.make_solver(c, shots=[c.shots[k]])
         single.run(0, 200)
         assert np.array_equal(single.seismograms(0), sol.seismograms(k)), k
+
+
+def test_acoustic3d_depth_that_leaves_no_even_parts():
+    """81 planes at order 2 ask for ten parts of nine planes, which nine parts already hold."""
+    _check(cases.acoustic_3d(NX=40, NY=81, NZ=36, NT=120, order=2))

@@ -421,7 +421,7 @@ int Elastic3D::run_adjoint()
     const Cpml3D P = cpml();
     const Acq Q = acq();
     const TapsT3D TT{a->tapT[0], a->tapT[1], a->tapT[2], a->tapT[3], a->tapT[4], a->tapT[5]};
-    const int adj_nyc = std::max(1, std::min(nyc, NY / std::max(4 * H, 8)));
+    const int adj_nyc = nyc;  // parts of at least max(4H, 8) planes (depth_parts)
     for (int seg = a->nck - 1; seg >= 0; seg--) {
         const int s0 = seg * a->every, s1 = std::min(NT, s0 + a->every);
         if ((rc = restore_checkpoint(seg))) return rc;

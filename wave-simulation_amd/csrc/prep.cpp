@@ -172,6 +172,13 @@ std::vector<double> abs_profile(int W, double damping_coeff)
     return c;
 }
 
+int depth_parts(int NY, int H, int tiles, int blocks)
+{
+    const int n = std::max(1, std::min((blocks + tiles - 1) / tiles, NY / std::max(4 * H, 8)));
+    const int planes = (NY + n - 1) / n;
+    return (NY + planes - 1) / planes;
+}
+
 void em_ca_cb(float eps, float sigma, float DT, float &ca, float &cb)
 {
     float q = 0.5f / eps;

@@ -57,4 +57,10 @@ void em_visco_coef(float eps_s, float sig_s, float tE, float tS, float DT, float
 // ABS damping factor of one grid cell (ABS2D.cpp:110-178, ABS3D.cpp:150-215).
 std::vector<double> abs_profile(int W, double damping_coeff);
 
+// Parts along depth that the 3D kernels deal NY planes into, equal ones of ceil(NY / parts)
+// planes: as many as bring `tiles` x-z tiles to `blocks` blocks, of at least 4H (and 8) planes
+// each, and none of them empty (a block of a part beyond the grid would load its window of
+// planes from beyond the field).
+int depth_parts(int NY, int H, int tiles, int blocks);
+
 }  // namespace wv

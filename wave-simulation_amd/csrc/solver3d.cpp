@@ -266,7 +266,7 @@ int Elastic3D::init(const wv_config &k, hipStream_t stream, int phys, bool visco
     }
     // chunks along y: enough blocks to fill the chip, chunks of at least 4H planes
     const int nxz = ((NX + TILE_X - 1) / TILE_X) * ((NZ + 4 * rz - 1) / (4 * rz)) * nshots;
-    nyc = std::max(1, std::min((kBlocks3D + nxz - 1) / nxz, NY / std::max(4 * H, 8)));
+    nyc = depth_parts(NY, H, nxz, kBlocks3D);
     HIP3(hipEventCreate(&ev0));
     HIP3(hipEventCreate(&ev1));
     shots.assign(nshots, Shot());
@@ -278,7 +278,7 @@ int Elastic3D::set_rz(int r)
 {
     rz = r;
     const int nxz = ((NX + TILE_X - 1) / TILE_X) * ((NZ + 4 * rz - 1) / (4 * rz)) * nshots;
-    nyc = std::max(1, std::min((kBlocks3D + nxz - 1) / nxz, NY / std::max(4 * H, 8)));
+    nyc = depth_parts(NY, H, nxz, kBlocks3D);
     acq_dirty = true;
     drop_graph();
     return 0;
