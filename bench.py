@@ -499,10 +499,11 @@ def main():
         "config": {"workload": "2D elastic P-SV order 8, 1000x1000, dx 1 m, dt 1e-4 s, 4000 steps, 30-cell CPML, "
                                "10 layers + 3% Gaussian perturbation, 1 VY Ricker 30 Hz shot, 1000 receivers "
                                "(one benchmark step = one shot)",
-                   "path": ("hand-written kernels, autotuned over single-pass, two-launch and row-strip variants"
+                   "path": ("hand-written kernels, autotuned over resident, single-pass, two-launch and row-strip variants"
                             if args.path == "fused" and args.tile_y == 0 else args.path),
                    "kernel": choice,
-                   "launches_per_time_step": 1 if choice.startswith("fused") else 2,
+                   "launches_per_time_step": (0 if choice == "resident" else  # one launch per shot
+                                              1 if choice.startswith("fused") else 2),
                    "steps_per_graph": args.graph, "shots_per_step": 1},
         # the step's algorithmic bytes over the whole timed loop (graphs, flushes, resets included)
         "hbm_frac_step": round(step_bytes * NT * args.steps / wall / 1e9 / HBM_PEAK_GBS, 4),

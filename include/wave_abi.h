@@ -47,8 +47,11 @@ extern "C" {
 #define WV_OPS_STENCIL 1 /* LAMA StencilMatrix: points outside the grid dropped (FDTD2D.cpp:156-185) */
 
 /* execution path */
-#define WV_PATH_FUSED 0  /* hand-written kernels, all shots per launch; one launch per time step
-                            where a single-pass kernel exists (2D elastic), else WV_PATH_PHASED */
+#define WV_PATH_FUSED 0  /* hand-written kernels, all shots per launch: with tile_y = 0 the two-launch
+                            kernels (2D elastic: the row-strip pair) and, for 2D acoustic, elastic, SH
+                            and TM-EM runs that fit, the resident loop (one cooperative launch per run
+                            call, fields in LDS; same results to the bit); with a tile_y the 2D elastic
+                            single-pass kernel (one launch per time step), else WV_PATH_PHASED */
 #define WV_PATH_PLAIN 1  /* reference operator sequence: CSR SpMV + vector passes, shot by shot */
 #define WV_PATH_PHASED 2 /* hand-written kernels, velocity-type and stress-type update as two launches */
 #define WV_PATH_STRIP 3  /* 2D elastic and TM-EM: two launches of row-strip kernels (each wavefront
@@ -159,7 +162,8 @@ int wv_set_wavefield(wv_solver *s, int shot, int field, const float *in);
  * resets the wavefields and seismograms.  *choice receives the index of the
  * variant kept (0..2 = two-launch with 8/16/32 rows, 3..5 = single pass with
  * 8/16/24 rows, 6..8 = 3D elastic with 4/8/16-row x-z tiles, 9..11 = 2D
- * elastic row-strip kernels with 8/16/32-row blocks, -1 = the handle has a
+ * elastic row-strip kernels with 8/16/32-row blocks, 12 = the persistent TM-EM
+ * kernel, 13 = the resident loop over the fastest two-launch kernels, -1 = the handle has a
  * single variant: WV_PATH_PLAIN).
  * No counterpart in the reference. */
 int wv_tune(wv_solver *s, int nsteps, int *choice);

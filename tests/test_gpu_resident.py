@@ -1,0 +1,109 @@
+"""The resident 2D time loop (resident2d_kernel.hpp) against the two-launch kernels.
+
+A handle that names no tile height may run its steps in the resident loop (fields in LDS, halos
+exchanged between blocks); a handle with an explicit tile height runs the two-launch kernels, which
+the other tests hold against the oracle.  Both do the same operations in the same order, so
+seismograms and final wavefields are equal to the bit: at tile edges (columns 63 .. 129), few and
+many rows, every order, CPML / ABS / rigid edges with and without a free surface, more sources than
+a wavefront and more receivers than a block holds, several rounds of shots, runs cut into pieces,
+and the adjoint's record.
+"""
+import numpy as np
+import pytest
+
+from wavesim import cases
+
+pytestmark = pytest.mark.gpu
+
+TWO = {"elastic": "strip", "acoustic": "phased", "sh": "phased", "tmem": "phased"}
+
+
+def _case(physics, NX, NY, NT, order, nshots, damping, fs=0, W=8, ops=None):
+    if physics == "elastic":
+        c = cases.visco_2d(NX=NX, NY=NY, NT=NT, nshots=nshots, order=order, W=W, damping=damping, free_surface=fs)
+        c.type, c.visco = "elastic", None
+    elif physics == "sh":
+        c = cases.sh_2d(NX=NX, NY=NY, NT=NT, nshots=nshots, order=order, W=W, damping=damping)
+    elif physics == "tmem":
+        c = cases.viscotmem_2d(NX=NX, NY=NY, NT=NT, nshots=nshots, order=order, W=W, damping=damping)
+        c.type, c.visco = "tmem", None
+    else:
+        c = cases.visco_2d(NX=NX, NY=NY, NT=NT, nshots=nshots, order=order, W=W, damping=damping, free_surface=fs)
+        c.type, c.visco, c.m1 = "acoustic", None, None
+    return c
+
+
+def _equal(c, NT, pieces=None, **kw):
+    a = cases.make_solver(c, **kw)
+    b = cases.make_solver(c, path=TWO[c.type], tile_y=16)
+    cuts = [0] + (pieces or []) + [NT]
+    for t0, t1 in zip(cuts[:-1], cuts[1:]):
+        a.run(t0, t1)
+    b.run(0, NT)
+    for k in range(len(c.shots)):
+        x, y = a.seismograms(k), b.seismograms(k)
+        assert np.abs(y).max() > 0
+        assert np.array_equal(x, y), (k, np.abs(x - y).max())
+        for f in range(5 if c.type == "elastic" else 3):
+            assert np.array_equal(a.wavefield(f, k), b.wavefield(f, k)), (k, f)
+
+
+@pytest.mark.parametrize("physics", ["elastic", "acoustic", "sh", "tmem"])
+@pytest.mark.parametrize("order,NX,NY,damping", [(2, 64, 40, 2), (4, 65, 33, 0), (6, 129, 97, 1), (8, 63, 150, 2),
+                                                 (8, 190, 41, 1), (10, 128, 61, 2), (12, 131, 130, 2)])
+def test_resident_equals_two_launch(physics, order, NX, NY, damping):
+    _equal(_case(physics, NX, NY, 90, order, 2, damping), 90)
+
+
+@pytest.mark.parametrize("physics", ["elastic", "acoustic"])
+@pytest.mark.parametrize("damping", [1, 2])
+def test_resident_free_surface(physics, damping):
+    _equal(_case(physics, 150, 70, 120, 8, 2, damping, fs=1), 120)
+
+
+@pytest.mark.parametrize("physics", ["elastic", "tmem"])
+def test_resident_run_in_pieces_and_stencil_operators(physics):
+    c = _case(physics, 100, 75, 100, 8, 1, 2)
+    a = cases.make_solver(c, ops_mode="stencil")
+    b = cases.make_solver(c, ops_mode="stencil", path=TWO[physics], tile_y=16)
+    for t0, t1 in ((0, 40), (40, 43), (43, 99), (99, 100)):
+        a.run(t0, t1)
+    b.run(0, 100)
+    assert np.array_equal(a.seismograms(0), b.seismograms(0))
+
+
+def test_resident_many_sources_and_receivers():
+    """More than 64 sources in one tile, on shared cells too, and more receivers than a block has threads."""
+    c = _case("elastic", 140, 90, 60, 8, 1, 2)
+    rng = np.random.default_rng(3)
+    sh = c.shots[0]
+    cells = np.concatenate([30 + np.arange(70) % 20 + (40 + np.arange(70) // 20) * 140, [30 + 40 * 140] * 5])
+    sh.src_index = cells
+    sh.src_type = np.array([1 + k % 3 for k in range(len(cells))], np.int32)
+    sh.src_signal = rng.standard_normal((len(cells), 60)).astype(np.float32)
+    sh.rec_index = np.tile(np.arange(20, 120) + 45 * 140, 25)
+    sh.rec_type = np.repeat([1, 2, 3, 2, 1], 500).astype(np.int32)
+    _equal(c, 60)
+
+
+def test_resident_rounds_of_shots():
+    """More shots than the chip holds at once: the blocks take them in rounds."""
+    _equal(_case("elastic", 300, 200, 200, 8, 23, 2), 200)
+
+
+def test_resident_record_gives_the_same_gradient():
+    """The record of the derivative sums written by the resident loop (rows per wavefront as the strips of
+    the record) leads to the gradient of the row-strip kernels' record."""
+    c = cases.elastic_c4(N=130, NT=120, nshots=3, W=10)
+    g = []
+    for ty in (16, 0):
+        sol = cases.make_solver(c, path="strip", tile_y=ty)
+        sol.set_checkpointing(40, True)
+        sol.run(0, 120)
+        for k in range(3):
+            sol.set_adjoint_source(k, sol.seismograms(k))
+        sol.run_adjoint()
+        g.append([sol.gradient(p) for p in ("vp", "vs", "rho")])
+    for x, y in zip(*g):
+        # (the adjoint pass adds its FP64 terms with atomics, in no fixed order)
+        assert np.linalg.norm(x - y) <= 1e-12 * np.linalg.norm(y)

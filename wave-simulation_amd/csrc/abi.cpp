@@ -40,6 +40,7 @@ wv_solver::~wv_solver()
     delete plain;
     delete e3;
     adjoint_destroy(adj);
+    res2d_destroy(this);
     free_list(acq_allocs);
     free_list(allocs);
     if (ev0) (void)hipEventDestroy(ev0);
@@ -53,6 +54,7 @@ int wv_solver::sync_acquisition()
     drop_graph();
     HIP_TRY(hipStreamSynchronize(st));
     free_list(acq_allocs);
+    res2d_acquisition_changed(this);
     std::vector<int> sp(1, 0), rp(1, 0), stp, rtp;
     std::vector<long long> sc, rc;
     std::vector<float> sig;
@@ -300,6 +302,9 @@ double wv_solver::kernel_bytes(int kind) const
     return bytes;
 }
 
+const char *const kResidentFailed =
+    "the resident time loop gave up waiting for its halos: the run's fields and seismograms are not valid";
+
 extern "C" {
 
 const char *wv_last_error(void) { return g_err.c_str(); }
@@ -448,6 +453,14 @@ int wv_init(wv_solver *s, const wv_config *c)
     // kernels index inside one field plane and one shot's CPML frame with 32-bit offsets
     if (L.plane >= (1LL << 31) || (long long)k.NY * k.NX >= (1LL << 30))
         return fail(WV_EINVAL, "grid too large for one field plane");
+    if (single && k.tile_y == 0 && wv::strip2d_fits(L)) {
+        // no tile height asked for: the row-strip pair, which the resident loop falls back to and
+        // which is faster than the single-pass kernel at every size measured (C2: 20.5 against
+        // 38.3 us per step)
+        s->variant = V_STRIP;
+        s->tile_x = wv::TILE_X;
+        s->tile_y = 16;
+    }
     if (s->variant == V_STRIP && !wv::strip2d_fits(L))
         return fail(WV_EINVAL, "grid too large for the row-strip kernels (field plane of 2 GiB or more)");
 
@@ -1009,6 +1022,10 @@ int wv_reset(wv_solver *s)
     return WV_OK;
 }
 
+// Shorter run segments stay with the two-launch kernels: a resident launch costs its set-up and one pass
+// over the state.
+static constexpr int kResidentSteps = 16;
+
 int wv_run(wv_solver *s, int t_start, int t_end)
 {
     if (!s || !s->inited) return fail(WV_ESTATE, "wv_run before wv_init");
@@ -1047,6 +1064,16 @@ int wv_run(wv_solver *s, int t_start, int t_end)
         if (ck && t % ck == 0 && (rc = adjoint_checkpoint(s, t))) return rc;
         int n = t_end - t;
         if (ck) n = std::min(n, ck - t % ck);
+        const wv::Rec2D *rec = adjoint_record(s);
+        if (n >= kResidentSteps && s->use_res && res2d_eligible(s) && (s->variant == V_STRIP || s->physics != wv::ELASTIC) &&
+            (s->use_res > 0 || res2d_expected(s, rec != nullptr))) {
+            const int r2 = res2d_run(s, t, n, rec);
+            if (r2 < 0) return r2;
+            if (r2 == 0) {
+                t += n;
+                continue;
+            }
+        }
         // (the persistent kernel is one cooperative launch per segment already: no graph)
         if (K > 0 && n >= K + s->cur && s->variant != V_PERSIST) {
             if (s->cur) {  // graphs start in buffer 0
@@ -1089,6 +1116,7 @@ int wv_synchronize(wv_solver *s)
 {
     if (!s || !s->inited) return fail(WV_ESTATE, "not initialised");
     HIP_TRY(hipStreamSynchronize(s->st));
+    if (res2d_failed(s)) return fail(WV_EDEVICE, kResidentFailed);
     return WV_OK;
 }
 
@@ -1122,6 +1150,7 @@ int wv_get_seismograms(wv_solver *s, int shot, float *out)
         return WV_OK;
     }
     HIP_TRY(hipStreamSynchronize(s->st));
+    if (res2d_failed(s)) return fail(WV_EDEVICE, kResidentFailed);
     std::vector<float> h((size_t)NT * s->rec_total);
     HIP_TRY(hipMemcpy(h.data(), s->d_seis, h.size() * sizeof(float), hipMemcpyDeviceToHost));
     const int r0 = s->rec_ptr_h[shot];
@@ -1147,6 +1176,7 @@ static int field_io(wv_solver *s, int shot, int field, float *out, const float *
     std::vector<float> h((size_t)L.plane);
     float *d = s->field[s->cur][field] + (size_t)shot * L.plane;
     HIP_TRY(hipStreamSynchronize(s->st));
+    if (res2d_failed(s)) return fail(WV_EDEVICE, kResidentFailed);
     if (out) {
         HIP_TRY(hipMemcpy(h.data(), d, h.size() * sizeof(float), hipMemcpyDeviceToHost));
         for (int y = 0; y < L.NY; y++)
@@ -1214,7 +1244,13 @@ int wv_tune(wv_solver *s, int nsteps, int *choice)
         if (rc) return rc;
         if ((rc = s->sync_acquisition())) return rc;
         wv::launch_set(s->d_tbase, 0, s->st);
-        if ((rc = s->enqueue_steps(2, false))) return rc;  // warm-up
+        rc = s->enqueue_steps(2, false);  // warm-up
+        if (rc && s->variant == V_PERSIST) {
+            // no cooperative launch to be had (one process at a time holds the GPU's cooperative queue)
+            (void)hipGetLastError();
+            continue;
+        }
+        if (rc) return rc;
         wv::launch_set(s->d_tbase, 0, s->st);
         HIP_TRY(hipEventRecord(s->ev0, s->st));
         if ((rc = s->enqueue_steps(nsteps, false))) return rc;
@@ -1234,6 +1270,39 @@ int wv_tune(wv_solver *s, int nsteps, int *choice)
     s->cur = 0;
     s->drop_graph();
     if (choice) *choice = cand_id[best_k];
+    if (!ck_every && res2d_eligible(s) && nsteps >= kResidentSteps) {
+        // the resident loop (for elastic over the row-strip pair, which takes its short segments)
+        const int v0 = s->variant, tx0 = s->tile_x, ty0 = s->tile_y;
+        if (s->physics == wv::ELASTIC && s->variant != V_STRIP && wv::strip2d_fits(s->L)) {
+            s->variant = V_STRIP;
+            s->tile_x = wv::TILE_X;
+            s->tile_y = 16;
+        }
+        s->use_res = 0;
+        int rc = wv_reset(s);
+        if (rc) return rc;
+        if ((rc = s->sync_acquisition())) return rc;
+        if (s->variant == V_STRIP || s->physics != wv::ELASTIC) {
+            if ((rc = res2d_run(s, 0, 2)) < 0) return rc;
+            if (rc == 0) {
+                HIP_TRY(hipEventRecord(s->ev0, s->st));
+                if ((rc = res2d_run(s, 0, nsteps)) < 0) return rc;
+                HIP_TRY(hipEventRecord(s->ev1, s->st));
+                HIP_TRY(hipEventSynchronize(s->ev1));
+                float ms = 0;
+                HIP_TRY(hipEventElapsedTime(&ms, s->ev0, s->ev1));
+                s->use_res = rc == 0 && ms < best ? 1 : 0;
+            }
+        }
+        if (s->use_res) {
+            if (choice) *choice = 13;
+        } else {
+            s->variant = v0;
+            s->tile_x = tx0;
+            s->tile_y = ty0;
+        }
+        s->acq_dirty = true;
+    }
     if (ck_every) {
         // the checkpoint / record layout depends on the kernel variant: lay it out
         // again for the variant kept (this also drops any earlier forward run)
@@ -1249,6 +1318,7 @@ int wv_set_kernel_timing(wv_solver *s, int on)
     if (!s || !s->inited) return fail(WV_ESTATE, "not initialised");
     if (s->plain) return fail(WV_EINVAL, "kernel timing is provided by the tiled kernels");
     s->ktiming = on != 0;
+    res2d_timing_reset(s);
     for (int k = 0; k < 7; k++) {
         s->kms[k] = 0;
         s->klaunch[k] = 0;
@@ -1285,6 +1355,7 @@ int wv_kernel_stats(wv_solver *s, int kind, const char **name, double *avg_ms, l
     }
     if (name)
         *name = kind >= 3 ? adj_names[kind - 3]
+                          : (res2d_timed(s) && kind < 2) ? (kind == 0 ? "res2d" : "-")
                           : ((s->variant == V_SINGLE && kind < 2)   ? (kind == 0 ? "el2d_fused" : "-")
                              : (s->variant == V_PERSIST && kind < 2) ? (kind == 0 ? "tm2d_persistent" : "")
                              : (s->variant == V_STRIP && kind < 2 && s->physics == wv::TMEM)
@@ -1294,7 +1365,9 @@ int wv_kernel_stats(wv_solver *s, int kind, const char **name, double *avg_ms, l
                                                                    : names[s->physics][kind]);
     if (launches) *launches = s->klaunch[kind];
     if (avg_ms) *avg_ms = s->klaunch[kind] ? s->kms[kind] / s->klaunch[kind] : 0.0;
-    if (bytes_per_launch) *bytes_per_launch = s->kernel_bytes(kind);
+    if (bytes_per_launch)
+        *bytes_per_launch = !res2d_timed(s) || kind > 1 ? s->kernel_bytes(kind)
+                            : (kind == 0 ? s->kernel_bytes(0) + s->kernel_bytes(1) : 0.0);
     return WV_OK;
 }
 

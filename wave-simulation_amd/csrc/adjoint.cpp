@@ -580,6 +580,7 @@ int wv_get_gradient(wv_solver *s, int param, double *out)
     const int NX = L.NX, NY = L.NY;
     const size_t n = (size_t)NX * NY;
     HIP_TRY(hipStreamSynchronize(s->st));
+    if (res2d_failed(s)) return fail(WV_EDEVICE, kResidentFailed);
     std::vector<double> g[5];
     std::vector<double> h((size_t)L.plane);
     for (int f = 0; f < 5; f++) {

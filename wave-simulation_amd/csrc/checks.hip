@@ -208,6 +208,7 @@ int wv_check_finite(wv_solver *s)
     unsigned h = 0;
     HIP_TRY(hipMemcpyAsync(&h, s->d_flag, sizeof(unsigned), hipMemcpyDeviceToHost, s->st));
     HIP_TRY(hipStreamSynchronize(s->st));
+    if (res2d_failed(s)) return fail(WV_EDEVICE, kResidentFailed);
     if (h) return fail(WV_ENONFINITE, NONFINITE_MSG);
     return WV_OK;
 }
@@ -235,6 +236,7 @@ int wv_check_finite_noalloc(wv_solver *s, long long *nonfinite)
     unsigned long long h[WV_NOALLOC_MAX_BUFFERS];
     HIP_TRY(hipMemcpyAsync(h, scr, sizeof(unsigned long long) * bufs.k, hipMemcpyDeviceToHost, s->st));
     HIP_TRY(hipStreamSynchronize(s->st));
+    if (res2d_failed(s)) return fail(WV_EDEVICE, kResidentFailed);
     unsigned long long total = 0;
     for (int k = 0; k < bufs.k; k++) total += h[k];
     if (nonfinite) *nonfinite = (long long)total;

@@ -42,6 +42,7 @@ struct ShotAcq {
 enum Variant { V_SINGLE = 0, V_PHASED = 1, V_STRIP = 2, V_PERSIST = 3 };
 
 struct AdjointState;
+struct Res2DState;
 
 struct wv_solver {
     int dim = 2;
@@ -103,6 +104,10 @@ struct wv_solver {
     hipGraphExec_t gexec = nullptr;
     int gsteps = 0;
 
+    // resident time loop (resident2d.cpp); use_res: -1 where the planner expects a gain, else as measured
+    // by wv_tune
+    Res2DState *res = nullptr;
+    int use_res = -1;
     // reference-sequence path
     wv::PlainSolver *plain = nullptr;
     // 3D elastic driver
@@ -294,3 +299,15 @@ const wv::Rec2D *adjoint_record(const wv_solver *s);
 void adjoint_run_begin(wv_solver *s, int t_start);
 int adjoint_checkpoint(wv_solver *s, int t);
 void adjoint_run_done(wv_solver *s, int t_end);
+
+// resident2d.cpp: the resident 2D time loop
+void res2d_destroy(wv_solver *s);
+void res2d_acquisition_changed(wv_solver *s);
+bool res2d_eligible(const wv_solver *s);
+int res2d_run(wv_solver *s, int t0, int nsteps, const wv::Rec2D *rec = nullptr, float *snap = nullptr,
+              long long snap_field = 0, long long snap_step = 0);
+bool res2d_expected(wv_solver *s, bool rec);
+bool res2d_failed(const wv_solver *s);
+extern const char *const kResidentFailed;
+bool res2d_timed(const wv_solver *s);  // the timed run calls went through the resident loop
+void res2d_timing_reset(wv_solver *s);

@@ -300,10 +300,8 @@ __global__ __launch_bounds__(NTHREADS) void ac2d_velocity(Layout2D L, Fields2D F
         if (col.xi >= 0) P.psx[0][((long long)shot * L.NY + y) * W2 + col.xi] = cpml(u, p0[r], col.axh, col.bxh);
         if (yi[r] >= 0) P.psy[0][((long long)shot * W2 + yi[r]) * L.NX + col.x] = cpml(t, q0[r], P.ayh[y], P.byh[y]);
         const long long o = L.at(col.x, y);
-        u *= crx[r];
-        vx[o] = ovx[r] + u;
-        t *= cry[r];
-        vy[o] = ovy[r] + t;
+        vx[o] = add_scaled(ovx[r], u, crx[r]);
+        vy[o] = add_scaled(ovy[r], t, cry[r]);
     }
 }
 
@@ -361,8 +359,7 @@ __global__ __launch_bounds__(NTHREADS) void ac2d_pressure(Layout2D L, Fields2D F
         if (col.xi >= 0) P.psx[1][((long long)shot * L.NY + y) * W2 + col.xi] = cpml(u, p1[r], col.ax, col.bx);
         if (yi[r] >= 0) P.psy[1][((long long)shot * W2 + yi[r]) * L.NX + col.x] = cpml(t, q1[r], P.ay[y], P.by[y]);
         u += t;
-        u *= cM[r];
-        float p = op[r] + u;
+        float p = add_scaled(op[r], u, cM[r]);
         p *= dmp[r];
         if (fs && y == 0) p *= 0.f;
         pr[L.at(col.x, y)] = p;
@@ -445,11 +442,8 @@ __device__ __forceinline__ void tm_h_tile(const Blk &B, const Layout2D &L, const
         if (col.xi >= 0) P.psx[0][((long long)shot * L.NY + y) * W2 + col.xi] = cpml(u2, p0[r], col.axh, col.bxh);
         // hx -= 1/mu_yz * CPML(Dyf ez) ; hy -= 1/mu_xz * (-CPML(Dxf ez))
         const long long o = L.at(col.x, y);
-        u *= cyz[r];
-        hx[o] = ohx[r] - u;
-        float w = -u2;
-        w *= cxz[r];
-        hy[o] = ohy[r] - w;
+        hx[o] = add_scaled(ohx[r], -u, cyz[r]);
+        hy[o] = add_scaled(ohy[r], u2, cxz[r]);
     }
 }
 
@@ -552,8 +546,7 @@ __device__ __forceinline__ void tm_e_tile(const Blk &B, const Layout2D &L, const
                     u -= V.dt * rn;
                 }
         }
-        u *= cb[r];
-        float e = ca[r] * oez[r] + u;
+        float e = tm_ez(ca[r], oez[r], cb[r], u);
         e *= dmp[r];
         ez[L.at(col.x, y)] = e;
     }
@@ -661,8 +654,7 @@ __global__ __launch_bounds__(NTHREADS) void sh2d_v(Layout2D L, Fields2D F, Coef2
         if (col.xi >= 0) P.psx[0][((long long)shot * L.NY + y) * W2 + col.xi] = cpml(u, p0[r], col.ax, col.bx);
         if (yi[r] >= 0) P.psy[0][((long long)shot * W2 + yi[r]) * L.NX + col.x] = cpml(t, q0[r], P.ay[y], P.by[y]);
         u += t;
-        u *= cr[r];
-        vz[L.at(col.x, y)] = ov[r] + u;
+        vz[L.at(col.x, y)] = add_scaled(ov[r], u, cr[r]);
     }
 }
 
@@ -719,10 +711,8 @@ __global__ __launch_bounds__(NTHREADS) void sh2d_s(Layout2D L, Fields2D F, Coef2
         if (col.xi >= 0) P.psx[1][((long long)shot * L.NY + y) * W2 + col.xi] = cpml(u, p1[r], col.axh, col.bxh);
         if (yi[r] >= 0) P.psy[1][((long long)shot * W2 + yi[r]) * L.NX + col.x] = cpml(t, q1[r], P.ayh[y], P.byh[y]);
         const long long o = L.at(col.x, y);
-        u *= cxz[r];
-        sxz[o] = (oxz[r] + u) * dmp[r];
-        t *= cyz[r];
-        syz[o] = (oyz[r] + t) * dmp[r];
+        sxz[o] = add_scaled(oxz[r], u, cxz[r]) * dmp[r];
+        syz[o] = add_scaled(oyz[r], t, cyz[r]) * dmp[r];
     }
     block_acquisition<SH>(A, F, so, shot_block(A, B), A.tbase[0] + tofs, false);
 }

@@ -1,0 +1,346 @@
+// Host side of the resident 2D time loop: launch plan, acquisition lists, exchange buffer, the
+// hand-shake with a launch.
+#include <sched.h>
+
+#include <algorithm>
+
+#include "handle.hpp"
+#include "resident2d_launch.hpp"
+
+namespace wv {
+
+hipError_t res2d_el(int order, bool rec, const void *go);
+hipError_t res2d_ac(int order, bool rec, const void *go);
+hipError_t res2d_tm(int order, bool rec, const void *go);
+hipError_t res2d_sh(int order, bool rec, const void *go);
+
+namespace {
+
+hipError_t res_dispatch(int physics, int order, bool rec, const ResGo &g)
+{
+    switch (physics) {
+    case ELASTIC: return res2d_el(order, rec, &g);
+    case ACOUSTIC: return res2d_ac(order, rec, &g);
+    case TMEM: return res2d_tm(order, rec, &g);
+    case SH: return res2d_sh(order, rec, &g);
+    default: return hipErrorInvalidValue;
+    }
+}
+
+size_t res_lds(int physics, int H, int rows)
+{
+    const int nf = physics == ELASTIC ? 5 : 3;
+    return sizeof(float) * ((size_t)nf * (rows + 2 * H) * (TILE_X + 2 * H) + 4ull * rows);
+}
+
+}  // namespace
+
+size_t res2d_words(int physics, int H, int rows, int *phase1)
+{
+    const int n = physics == ELASTIC ? 2 : 1, rpg = TILE_X / H;
+    const int items = 2 * n * ((rows + rpg - 1) / rpg) + 2 * n * H;
+    *phase1 = items * 64;
+    return (size_t)2 * items * 64;
+}
+
+static int wv_cu_count()
+{
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+        return 0;
+    return cus;
+}
+
+// Blocks of a plan that the device holds at once (0: the plan does not launch there).
+static int res_capacity(int physics, int order, const Res2DPlan &p, bool rec)
+{
+    int cap = 0;
+    ResGo g{};
+    g.plan = &p;
+    g.capacity = &cap;
+    g.lds = res_lds(physics, order / 2, p.srow * p.wmax);
+    if (res_dispatch(physics, order, rec, g) != hipSuccess) {
+        (void)hipGetLastError();
+        return 0;
+    }
+    // a block whose wavefronts do not spread evenly over the four SIMDs of a CU may find no place beside
+    // another one although registers and LDS would do in sum: count one block per CU then
+    return p.nwv % 4 ? std::min(cap, wv_cu_count()) : cap;
+}
+
+// Estimated us per time step of the whole batch: rounds x (exchange, barriers and latency of a step +
+// the arithmetic of the rows a CU holds).  Measured (MI355X, order 8; us per round): elastic 64 rows
+// per CU 11.9 (one block of 16 x 4 rows) and 12.4 (two of 8 x 4), 16 rows 5.7; TM-EM 64 rows 6.4 - 6.7;
+// SH 64 rows 6.0, 128 rows 10.4; acoustic order 4: 4 rows 3.5, 64 rows 4.7.
+static double res_step_us(int physics, int order, const Res2DPlan &p, int nshots)
+{
+    const int rounds = (nshots + p.conc - 1) / p.conc, cus = std::max(1, wv_cu_count());
+    const double rows = (double)p.rows() * ((p.blocks() + cus - 1) / cus);
+    const double per_row = (physics == ELASTIC ? 0.13 : 0.052) * (order + 4) / 12.0;
+    return rounds * (3.3 + 0.1 * p.srow + per_row * rows * (p.srow == 8 ? 1.2 : 1.0));
+}
+
+// The same of the two-launch kernels: launch gaps and one memory round trip per phase, then their
+// traffic.  Measured (us): elastic 1e6 cells 21.8, 1.44e6 31.4, 8e6 107; TM-EM 5.1e6 46, 2.05e7 195;
+// SH 0.94e6 15.8; acoustic 4e4 7.5 - 10.5.
+static double two_launch_us(int physics, double cells)
+{
+    return 7.0 + cells * (physics == ELASTIC ? 1.3e-5 : 9.1e-6);
+}
+
+// srow != 0: that many rows per wavefront, with the record of the derivative sums
+Res2DPlan res2d_plan(int physics, int order, const Layout2D &L, int nshots, int srow, double *gain)
+{
+    Res2DPlan best;
+    *gain = 0.0;
+    if (physics != ELASTIC && physics != ACOUSTIC && physics != TMEM && physics != SH) return best;
+    const int H = order / 2;
+    double best_t = 1e30;
+    static const int variants[5][2] = {{1, 16}, {2, 16}, {4, 16}, {4, 8}, {8, 8}};
+    for (auto &va : variants) {
+        const int S = va[0], wmax = va[1];
+        if (srow && S != srow) continue;
+        if (res_lds(physics, H, S * wmax) + 1024 > 160 * 1024) continue;
+        int cap[17] = {};
+        for (int w = 1; w <= wmax; w++) {
+            Res2DPlan p;
+            p.nwv = w;
+            p.srow = S;
+            p.wmax = wmax;
+            const int R = p.rows();
+            if (R < H) continue;  // a halo reaches into the next tile only
+            p.nbx = (L.NX + TILE_X - 1) / TILE_X;
+            p.nby = (L.NY + R - 1) / R;
+            p.conc = 1;
+            const long long per = (long long)p.nbx * p.nby;
+            if (per > 4096) continue;
+            cap[w] = res_capacity(physics, order, p, srow != 0);
+            if (per > cap[w]) continue;
+            const int most = cap[w] / (int)per, rounds = (nshots + most - 1) / most;
+            p.conc = (nshots + rounds - 1) / rounds;
+            const double t = res_step_us(physics, order, p, nshots);
+            if (t < best_t) {
+                best_t = t;
+                best = p;
+            }
+        }
+    }
+    if (best) *gain = two_launch_us(physics, (double)L.NX * L.NY * nshots) / best_t;
+    return best;
+}
+
+hipError_t launch_res2d(int physics, int order, const Res2DPlan &plan, const Layout2D &L, const Fields2D &F,
+                        const Coef2D &C, const Taps &T, const Cpml2D &P, const Acq &A, const Res2DArgs &X,
+                        const Rec2D *rec, hipStream_t stream)
+{
+    ResGo g{};
+    g.plan = &plan;
+    g.L = &L;
+    g.F = &F;
+    g.C = &C;
+    g.T = &T;
+    g.P = &P;
+    g.A = &A;
+    g.X = &X;
+    g.rec = rec ? *rec : Rec2D{};
+    g.st = stream;
+    g.lds = res_lds(physics, order / 2, plan.srow * plan.wmax);
+    return res_dispatch(physics, order, rec != nullptr || X.snap != nullptr, g);
+}
+
+}  // namespace wv
+
+struct Res2DState {
+    wv::Res2DPlan plan;
+    double gain = 0.0;  // estimated step time of the two-launch kernels over that of the plan
+    bool planned = false, lists = false;
+    int srow = 0;
+    std::vector<void *> allocs;      // exchange buffer, control words
+    std::vector<void *> acq_allocs;  // lists of the plan's tiles
+    int *bsrc_ptr = nullptr, *bsrc = nullptr, *brec_ptr = nullptr, *brec = nullptr;
+    unsigned long long *xch = nullptr;
+    unsigned *ctl = nullptr;
+    float *psi = nullptr;
+    unsigned *host = nullptr;  // pinned
+    int words = 0, phase1 = 0;  // exchange words of a block
+    unsigned tag = 1, arrived = 0, launches = 0;
+    hipEvent_t ev[2] = {};  // per-kernel timing
+    bool timed = false;     // the timed run calls went through the resident loop
+};
+
+void res2d_destroy(wv_solver *s)
+{
+    if (!s->res) return;
+    s->free_list(s->res->acq_allocs);
+    s->free_list(s->res->allocs);
+    if (s->res->host) (void)hipHostFree(s->res->host);
+    for (hipEvent_t e : s->res->ev)
+        if (e) (void)hipEventDestroy(e);
+    delete s->res;
+    s->res = nullptr;
+}
+
+void res2d_acquisition_changed(wv_solver *s)
+{
+    if (!s->res) return;
+    s->free_list(s->res->acq_allocs);
+    s->res->lists = false;
+}
+
+bool res2d_eligible(const wv_solver *s)
+{
+    if (s->dim != 2 || s->plain || s->visco) return false;
+    if (s->physics != wv::ELASTIC && s->physics != wv::ACOUSTIC && s->physics != wv::TMEM && s->physics != wv::SH)
+        return false;
+    return s->cfg.tile_y == 0 && (s->cfg.path == WV_PATH_FUSED || (s->cfg.path == WV_PATH_STRIP && s->physics == wv::ELASTIC));
+}
+
+// The plan for the handle (rows per wavefront as the record's strips when it is written); false:
+// the resident loop does not take this problem.
+static bool res_plan(wv_solver *s, int srow)
+{
+    if (!s->res) s->res = new Res2DState();
+    Res2DState *r = s->res;
+    if (r->planned && r->srow == srow) return (bool)r->plan;
+    s->free_list(r->acq_allocs);
+    s->free_list(r->allocs);
+    r->lists = false;
+    r->plan = wv::res2d_plan(s->physics, s->cfg.spatial_fd_order, s->L, s->cfg.nshots, srow, &r->gain);
+    r->planned = true;
+    r->srow = srow;
+    r->xch = nullptr;
+    r->ctl = nullptr;
+    r->tag = 1;
+    r->arrived = r->launches = 0;
+    return (bool)r->plan;
+}
+
+// nsteps steps from t0 in one launch.  0: done (enqueued and started); 1: not started (the caller
+// runs the steps with the ordinary kernels); < 0: error.
+int res2d_run(wv_solver *s, int t0, int nsteps, const wv::Rec2D *rec, float *snap, long long snap_field,
+              long long snap_step)
+{
+    if (!res_plan(s, rec || snap ? s->tile_y / 4 : 0)) return 1;
+    Res2DState *r = s->res;
+    const wv::Res2DPlan &p = r->plan;
+    int rc;
+    if (!r->xch) {
+        r->words = (int)wv::res2d_words(s->physics, s->H, p.rows(), &r->phase1);
+        if ((rc = s->dalloc(&r->xch, (size_t)r->words * p.blocks(), r->allocs)) || (rc = s->dalloc(&r->ctl, 3, r->allocs)) ||
+            (s->cfg.damping_boundary == 2 &&
+             (rc = s->dalloc(&r->psi, (size_t)p.blocks() * p.nwv * 4 * (s->physics == wv::ELASTIC ? 2 : 1) * p.srow * 64,
+                             r->allocs))))
+            return rc;
+        if (!r->host) HIP_TRY(hipHostMalloc((void **)&r->host, 64, hipHostMallocDefault));
+        r->host[0] = r->host[1] = 0;
+    }
+    if (!r->lists) {
+        const int R = p.rows();
+        const size_t nsb = (size_t)s->cfg.nshots * p.nby * p.nbx;
+        std::vector<std::vector<int>> bs(nsb), br(nsb);
+        int gs = 0, gr = 0;
+        for (int sh = 0; sh < s->cfg.nshots; sh++) {
+            auto blk = [&](long long g) {
+                const int x = (int)(g % s->L.NX), y = (int)(g / s->L.NX);
+                return ((size_t)sh * p.nby + y / R) * p.nbx + x / wv::TILE_X;
+            };
+            for (long long g : s->shots[sh].sidx) bs[blk(g)].push_back(gs++);
+            for (long long g : s->shots[sh].ridx) br[blk(g)].push_back(gr++);
+        }
+        std::vector<int> bsp(1, 0), bsl, brp(1, 0), brl;
+        for (size_t b = 0; b < nsb; b++) {
+            bsl.insert(bsl.end(), bs[b].begin(), bs[b].end());
+            bsp.push_back((int)bsl.size());
+            brl.insert(brl.end(), br[b].begin(), br[b].end());
+            brp.push_back((int)brl.size());
+        }
+        if ((rc = s->upload(&r->bsrc_ptr, bsp, r->acq_allocs)) || (rc = s->upload(&r->bsrc, bsl, r->acq_allocs)) ||
+            (rc = s->upload(&r->brec_ptr, brp, r->acq_allocs)) || (rc = s->upload(&r->brec, brl, r->acq_allocs)))
+            return rc;
+        r->lists = true;
+    }
+    wv::Res2DArgs X{};
+    X.nwv = p.nwv;
+    X.nbx = p.nbx;
+    X.nby = p.nby;
+    X.conc = p.conc;
+    X.nshots = s->cfg.nshots;
+    X.t0 = t0;
+    X.nsteps = nsteps;
+    X.words = r->words;
+    X.phase1 = r->phase1;
+    X.xch = r->xch;
+    X.tag0 = r->tag;
+    X.ctl = r->ctl;
+    X.launch = ++r->launches;
+    r->arrived += (unsigned)p.blocks();
+    X.arrive = r->arrived;
+    X.host = r->host;
+    X.bsrc_ptr = r->bsrc_ptr;
+    X.bsrc = r->bsrc;
+    X.brec_ptr = r->brec_ptr;
+    X.brec = r->brec;
+    X.psi = r->psi;
+    X.snap = snap;
+    X.snap_field = snap_field;
+    X.snap_step = snap_step;
+    hipEvent_t e0 = nullptr, e1 = nullptr;
+    if (s->ktiming) {
+        for (auto &ev : r->ev)
+            if (!ev) HIP_TRY(hipEventCreate(&ev));
+        e0 = r->ev[0];
+        e1 = r->ev[1];
+        r->timed = true;
+        HIP_TRY(hipEventRecord(e0, s->st));
+    }
+    const hipError_t e = wv::launch_res2d(s->physics, s->cfg.spatial_fd_order, p, s->L, s->fields2d(s->cur), s->coef2d(),
+                                          s->taps(), s->cpml2d(s->cur), s->acq(), X, rec, s->st);
+    if (e != hipSuccess) {
+        // nothing ran: leave the counters as the device has them
+        r->launches--;
+        r->arrived -= (unsigned)p.blocks();
+        (void)hipGetLastError();
+        return 1;
+    }
+    const int rounds = (s->cfg.nshots + p.conc - 1) / p.conc;
+    r->tag += (unsigned)(rounds * nsteps);
+    // the launch says whether all its blocks came in before it touched the state
+    volatile unsigned *h = r->host;
+    const unsigned go = 2 * X.launch, stop = go + 1;
+    for (int n = 1; h[0] != go && h[0] != stop; n++) {
+        if ((n & 255) == 0) {
+            const hipError_t q = hipStreamQuery(s->st);
+            if (q != hipSuccess && q != hipErrorNotReady) HIP_TRY(q);
+            if (q == hipSuccess && h[0] != go && h[0] != stop)
+                return fail(WV_EDEVICE, "the resident time loop ended without a verdict");
+        }
+        sched_yield();
+    }
+    if (h[0] == go) {
+        if (e0) {
+            HIP_TRY(hipEventRecord(e1, s->st));
+            HIP_TRY(hipEventSynchronize(e1));
+            float ms = 0;
+            HIP_TRY(hipEventElapsedTime(&ms, e0, e1));
+            s->kms[0] += ms;
+            s->klaunch[0] += nsteps;  // counted per time step
+        }
+        return 0;
+    }
+    // something else holds the GPU: this handle stays with the ordinary kernels from here on
+    r->plan = wv::Res2DPlan{};
+    return 1;
+}
+
+// Whether the planner expects the resident loop to be the faster one for the handle's run calls.
+bool res2d_expected(wv_solver *s, bool rec) { return res_plan(s, rec ? s->tile_y / 4 : 0) && s->res->gain > 1.05; }
+
+// A wait inside a resident launch ran out (checked where results are handed out).
+bool res2d_failed(const wv_solver *s) { return s->res && s->res->host && ((volatile unsigned *)s->res->host)[1]; }
+
+bool res2d_timed(const wv_solver *s) { return s->res && s->res->timed; }
+void res2d_timing_reset(wv_solver *s)
+{
+    if (s->res) s->res->timed = false;
+}

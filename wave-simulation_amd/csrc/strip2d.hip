@@ -22,25 +22,13 @@
 //     the planes carry no vector address arithmetic.
 // Sources and receivers use the per-(shot, block) lists of the tiled kernels
 // with 4S-row blocks.
-#include <hip/hip_fp16.h>
-
-#include "acq2d.hpp"
+#include "strip2d.hpp"
 
 namespace wv {
 namespace {
 
 // byte offset of (x, y) in a padded plane (planes are below 2 GiB: checked by the launcher)
 __device__ __forceinline__ int boff(const Layout2D &L, int x, int y) { return (int)(L.at(x, y) * 4); }
-
-// general form: table taps for offsets -H..H
-template <int K>
-__device__ __forceinline__ float dtab(const float *v, const float *c)
-{
-    float s = 0.f;
-#pragma unroll
-    for (int k = 0; k < K; k++) s += c[k] * v[k];
-    return s;
-}
 
 // Per-array buffer resources and lane offsets of one wavefront's strip.
 struct StripCtx {
@@ -69,59 +57,6 @@ __device__ __forceinline__ StripCtx strip_ctx(const Layout2D &L, const Cpml2D &P
     c.vxi = (unsigned)col.xi * 4u;
     c.vl = (unsigned)c.lane * 4u;
     return c;
-}
-
-// Record NF fields (f0, f0+1, ...) of the wavefront's strip (S rows x 64
-// columns) for the adjoint pass (Rec2D): the maximum over the strip (a DPP
-// wavefront reduction) sets each field's FP16 scale; rows are stored in pairs,
-// one 32-bit word per lane and pair.
-template <int S, int NF>
-__device__ __forceinline__ void record_strips(const Rec2D &R, const Layout2D &L, int nshots, int t, int f0, int shot,
-                                              int x0, int ya, int lane, const float (&h)[NF][S])
-{
-    static_assert(S % 2 == 0, "rows are recorded in pairs");
-    const bool in = x0 + lane < L.NX;
-    float m[NF];
-#pragma unroll
-    for (int f = 0; f < NF; f++) {
-        m[f] = 0.f;
-#pragma unroll
-        for (int r = 0; r < S; r++)
-            if (in && ya + r < L.NY) m[f] = fmaxf(m[f], fabsf(h[f][r]));
-    }
-#pragma unroll
-    for (int f = 0; f < NF; f++) m[f] = wave_max_nonneg(m[f]);
-    if (ya >= L.NY) return;  // a strip wholly below the grid (last block row) records nothing
-#pragma unroll
-    for (int f = 0; f < NF; f++) {
-        // strips whose values are all below 1e-30 are stored as zeros (scale 1); above it the
-        // scale stays a normal float, so h / scale is finite
-        const float sc = m[f] > 1e-30f ? m[f] * (1.f / 32768.f) : 1.f, is = 1.f / sc;
-        const long long fs = ((long long)t * 5 + f0 + f) * nshots + shot;
-        const long long q = (fs * R.nty + ya / S) * R.nbx + x0 / TILE_X;
-        if (lane == 0) R.scale[q] = sc;
-        unsigned *w = R.h + q * (S / 2) * TILE_X + lane;
-#pragma unroll
-        for (int p = 0; p < S / 2; p++) {
-            // cells outside the grid store zeros
-            const float a = (in && ya + 2 * p < L.NY) ? h[f][2 * p] * is : 0.f;
-            const float b = (in && ya + 2 * p + 1 < L.NY) ? h[f][2 * p + 1] * is : 0.f;
-            // written once, read once much later: streamed past the caches
-            __builtin_nontemporal_store((unsigned)__half_as_ushort(__float2half_rn(a)) |
-                                            ((unsigned)__half_as_ushort(__float2half_rn(b)) << 16),
-                                        w + p * TILE_X);
-        }
-    }
-}
-
-// y derivative at window row i (own row) with the row's table taps c (offsets -H..H)
-template <int H, int N>
-__device__ __forceinline__ float ydiff(const float (&w)[N], int i, const float *c)
-{
-    float s = 0.f;
-#pragma unroll
-    for (int k = 0; k <= 2 * H; k++) s += c[k] * w[i + k - H];
-    return s;
 }
 
 // The y taps of this wavefront's S rows (two tables) and the rows' CPML y
@@ -290,10 +225,8 @@ __global__ __launch_bounds__(NTHREADS) void el2d_velocity_strip(Layout2D L, Fiel
                 Sn.h[0][c.so + L.at(c.x0, y) + lane] = u;
                 Sn.h[1][c.so + L.at(c.x0, y) + lane] = u2;
             }
-            u *= crx[r];
-            u2 *= cry[r];
-            bstore(ovx[r] + u, bvx, c.vc, ro);
-            bstore(ovy[r] + u2, bvy, c.vc, ro);
+            bstore(add_scaled(ovx[r], u, crx[r]), bvx, c.vc, ro);
+            bstore(add_scaled(ovy[r], u2, cry[r]), bvy, c.vc, ro);
         }
         wave_sync();
     }
@@ -422,12 +355,7 @@ __global__ __launch_bounds__(NTHREADS) void el2d_stress_strip(Layout2D L, Fields
                 py3[yi * L.NX + c.x0 + lane] = cpml(u2, q3[r], cy[3], cy[4]);
             }
             float xx = oxx[r], yy = oyy[r], xy = oxy[r];
-            float u = a1 + a3;
-            u *= cM[r];
-            xx += u;
-            yy += u;
-            xx -= 2.f * (a3 * cmu[r]);
-            yy -= 2.f * (a1 * cmu[r]);
+            el_normal(xx, yy, a1, a3, cM[r], cmu[r]);
             u2 += a2;
             rh[0][r] = a1;
             rh[1][r] = a3;
@@ -438,14 +366,8 @@ __global__ __launch_bounds__(NTHREADS) void el2d_stress_strip(Layout2D L, Fields
                 Sn.h[3][hr] = a3;
                 Sn.h[4][hr] = u2;
             }
-            u2 *= cmxy[r];
-            xy += u2;
-            if (fs && y == 0) {
-                // FreeSurface2Delastic.cpp:14-45, FreeSurface.cpp:14-21
-                xx += C.fsH[col.x] * a1;
-                xx -= C.fsV[col.x] * a3;
-                yy *= 0.f;
-            }
+            xy = add_scaled(xy, u2, cmxy[r]);
+            if (fs && y == 0) el_surface(xx, yy, a1, a3, C.fsH[col.x], C.fsV[col.x]);
             xx *= dmp[r];
             yy *= dmp[r];
             xy *= dmp[r];
@@ -545,11 +467,8 @@ __global__ __launch_bounds__(NTHREADS) void tm2d_h_strip(Layout2D L, Fields2D F,
                 py0[yi * L.NX + c.x0 + lane] = cpml(u, q0[r], cy[2], cy[3]);
             }
             const int ro = boff(L, c.xl, y);
-            u *= cyz[r];
-            bstore(ohx[r] - u, bhx, c.vc, ro);
-            float w = -u2;
-            w *= cxz[r];
-            bstore(ohy[r] - w, bhy, c.vc, ro);
+            bstore(add_scaled(ohx[r], -u, cyz[r]), bhx, c.vc, ro);
+            bstore(add_scaled(ohy[r], u2, cxz[r]), bhy, c.vc, ro);
         }
         wave_sync();
     }
@@ -636,8 +555,7 @@ __global__ __launch_bounds__(NTHREADS) void tm2d_e_strip(Layout2D L, Fields2D F,
                 py1[yi * L.NX + c.x0 + lane] = cpml(t, q1[r], cy[0], cy[1]);
             }
             u -= t;
-            u *= cb[r];
-            float e = ca[r] * oez[r] + u;
+            float e = tm_ez(ca[r], oez[r], cb[r], u);
             e *= dmp[r];
             bstore(e, bez, c.vc, boff(L, c.xl, y));
         }

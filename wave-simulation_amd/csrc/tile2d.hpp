@@ -103,7 +103,7 @@ __device__ __forceinline__ float dx(const float (*S)[RW], int r, int tx, const f
 {
     float s = 0.f;
 #pragma unroll
-    for (int k = 0; k <= 2 * H; k++) s += c[k] * S[r][tx + k];
+    for (int k = 0; k <= 2 * H; k++) s = __builtin_fmaf(c[k], S[r][tx + k], s);
     return s;
 }
 
@@ -113,17 +113,38 @@ __device__ __forceinline__ float dy(const float (*S)[RW], int r, int tx, const f
 {
     float s = 0.f;
 #pragma unroll
-    for (int k = 0; k <= 2 * H; k++) s += c[k] * S[r + k - H][tx + H];
+    for (int k = 0; k <= 2 * H; k++) s = __builtin_fmaf(c[k], S[r + k - H][tx + H], s);
     return s;
 }
 
-// psi = b*psi + a*d ; d += psi   (CPML.cpp:84-95)
+// psi = b*psi + a*d ; d += psi   (CPML.cpp:84-95); the rounding is spelled out, so every kernel
+// that shares this gives the same bits
 __device__ __forceinline__ float cpml(float &d, float psi, float a, float b)
 {
-    float p = b * psi;
-    p = p + a * d;
+    const float p = __builtin_fmaf(a, d, b * psi);
     d = d + p;
     return p;
+}
+
+// Cell updates with their rounding spelled out, for the kernels whose runs change over to one another
+// at any step: a field plus coefficient times derivative sum, TM-EM Ca ez + Cb (curl), and the
+// normal stresses of P-SV (a1 = Dx vx, a3 = Dy vy).
+__device__ __forceinline__ float add_scaled(float f, float d, float c) { return __builtin_fmaf(d, c, f); }
+__device__ __forceinline__ float tm_ez(float ca, float ez, float cb, float curl)
+{
+    return __builtin_fmaf(ca, ez, curl * cb);
+}
+__device__ __forceinline__ void el_normal(float &xx, float &yy, float a1, float a3, float M, float mu)
+{
+    const float s = a1 + a3;
+    xx = __builtin_fmaf(-2.f, a3 * mu, __builtin_fmaf(s, M, xx));
+    yy = __builtin_fmaf(-2.f, a1 * mu, __builtin_fmaf(s, M, yy));
+}
+// the surface row (FreeSurface2Delastic.cpp:14-45, FreeSurface.cpp:14-21)
+__device__ __forceinline__ void el_surface(float &xx, float &yy, float a1, float a3, float fsH, float fsV)
+{
+    xx = __builtin_fmaf(-fsV, a3, __builtin_fmaf(fsH, a1, xx));
+    yy *= 0.f;
 }
 
 struct Col {

@@ -129,7 +129,7 @@ class ForwardSolver:
         _abi.check(_abi.load().wv_run(self._h, int(t_start), int(t_end)))
 
     TUNE_CHOICES = ("phased-8", "phased-16", "phased-32", "fused-8", "fused-16", "fused-24", "3d-z4", "3d-z8",
-                    "3d-z16", "strip-8", "strip-16", "strip-32", "persistent-16")
+                    "3d-z16", "strip-8", "strip-16", "strip-32", "persistent-16", "resident")
 
     def tune(self, nsteps=100):
         """Time every kernel variant on this problem, keep the fastest (resets the wavefields)."""
