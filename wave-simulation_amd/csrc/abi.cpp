@@ -1151,11 +1151,7 @@ int wv_get_seismograms(wv_solver *s, int shot, float *out)
     }
     HIP_TRY(hipStreamSynchronize(s->st));
     if (res2d_failed(s)) return fail(WV_EDEVICE, kResidentFailed);
-    std::vector<float> h((size_t)NT * s->rec_total);
-    HIP_TRY(hipMemcpy(h.data(), s->d_seis, h.size() * sizeof(float), hipMemcpyDeviceToHost));
-    const int r0 = s->rec_ptr_h[shot];
-    for (int r = 0; r < nrec; r++)
-        for (int t = 0; t < NT; t++) out[(size_t)r * NT + t] = h[(size_t)t * s->rec_total + r0 + r];
+    HIP_TRY(wv::read_traces(s->stage, s->d_seis, s->rec_total, s->rec_ptr_h[shot], nrec, NT, out, s->st));
     return WV_OK;
 }
 
@@ -1173,16 +1169,13 @@ static int field_io(wv_solver *s, int shot, int field, float *out, const float *
     }
     if (field < 0 || field >= s->nfields) return fail(WV_EINVAL, "bad field index");
     const wv::Layout2D &L = s->L;
-    std::vector<float> h((size_t)L.plane);
     float *d = s->field[s->cur][field] + (size_t)shot * L.plane;
     HIP_TRY(hipStreamSynchronize(s->st));
     if (res2d_failed(s)) return fail(WV_EDEVICE, kResidentFailed);
     if (out) {
-        HIP_TRY(hipMemcpy(h.data(), d, h.size() * sizeof(float), hipMemcpyDeviceToHost));
-        for (int y = 0; y < L.NY; y++)
-            for (int x = 0; x < L.NX; x++) out[(size_t)y * L.NX + x] = h[(size_t)L.at(x, y)];
+        HIP_TRY(wv::read_grid(s->stage, d, s->grid(), out, s->st));
     } else {
-        std::fill(h.begin(), h.end(), 0.f);
+        std::vector<float> h((size_t)L.plane, 0.f);
         for (int y = 0; y < L.NY; y++)
             for (int x = 0; x < L.NX; x++) h[(size_t)L.at(x, y)] = in[(size_t)y * L.NX + x];
         HIP_TRY(hipMemcpy(d, h.data(), h.size() * sizeof(float), hipMemcpyHostToDevice));

@@ -581,79 +581,15 @@ int wv_get_gradient(wv_solver *s, int param, double *out)
     const size_t n = (size_t)NX * NY;
     HIP_TRY(hipStreamSynchronize(s->st));
     if (res2d_failed(s)) return fail(WV_EDEVICE, kResidentFailed);
-    std::vector<double> g[5];
-    std::vector<double> h((size_t)L.plane);
-    for (int f = 0; f < 5; f++) {
-        HIP_TRY(hipMemcpy(h.data(), a->grad[f], h.size() * sizeof(double), hipMemcpyDeviceToHost));
-        g[f].resize(n);
-        for (int y = 0; y < NY; y++)
-            for (int x = 0; x < NX; x++) g[f][(size_t)y * NX + x] = h[(size_t)L.at(x, y)];
-    }
+    // coefficients (params 3..7) as they are; vp, vs, rho by the chain rule on the device (FP64)
     if (param >= 3) {
-        std::memcpy(out, g[param - 3].data(), n * sizeof(double));
+        HIP_TRY(wv::read_grid(s->stage, a->grad[param - 3], s->grid(), out, s->st));
         return WV_OK;
     }
-    // chain rule: coefficients (Modelparameter.cpp:336-639 rules) -> vp, vs, rho
-    const std::vector<float> &vp = s->model_h[0], &vs = s->model_h[1], &rho = s->model_h[2];
-    if (vp.size() != n) return fail(WV_ESTATE, "model not retained");
-    auto gi = [&](int x, int y) { return (size_t)y * NX + x; };
-    std::vector<double> mu(n), gmu(g[3]), gvp(n, 0.0), gvs(n, 0.0), grho(n, 0.0);
-    for (size_t i = 0; i < n; i++) mu[i] = std::max((double)rho[i] * vs[i] * vs[i], 1.0);
-    for (int y = 0; y < NY; y++)
-        for (int x = 0; x < NX; x++) {
-            const size_t j = gi(x, y);
-            const bool inx = x + 1 < NX, iny = y + 1 < NY;
-            size_t pts[4];
-            int npt = 0;
-            double w;
-            pts[npt++] = j;
-            if (inx && iny) {
-                pts[npt++] = gi(x + 1, y);
-                pts[npt++] = gi(x, y + 1);
-                pts[npt++] = gi(x + 1, y + 1);
-                w = 0.25;
-            } else if (inx) {
-                pts[npt++] = gi(x + 1, y);
-                w = 0.5;
-            } else if (iny) {
-                pts[npt++] = gi(x, y + 1);
-                w = 0.5;
-            } else {
-                w = 1.0;
-            }
-            double avg = 0;
-            for (int q = 0; q < npt; q++) avg += 1.0 / mu[pts[q]];
-            const double mxy = 1.0 / (w * avg);
-            if (mxy < 4.0) continue;  // mu_xy set to 0: no dependence
-            for (int q = 0; q < npt; q++) gmu[pts[q]] += g[4][j] * mxy * mxy * w / (mu[pts[q]] * mu[pts[q]]);
-        }
-    for (int y = 0; y < NY; y++)
-        for (int x = 0; x < NX; x++) {
-            const size_t i = gi(x, y);
-            const double r = rho[i], p = vp[i], v = vs[i];
-            gvp[i] = g[2][i] * 2.0 * r * p;
-            grho[i] += g[2][i] * p * p;
-            if (r * v * v >= 1.0) {
-                gvs[i] = gmu[i] * 2.0 * r * v;
-                grho[i] += gmu[i] * v * v;
-            }
-            if (x + 1 < NX) {
-                const double ix = 2.0 / (r + (double)rho[gi(x + 1, y)]);
-                grho[i] += g[0][i] * (-0.5 * ix * ix);
-                grho[gi(x + 1, y)] += g[0][i] * (-0.5 * ix * ix);
-            } else {
-                grho[i] += g[0][i] * (-1.0 / (r * r));
-            }
-            if (y + 1 < NY) {
-                const double iy = 2.0 / (r + (double)rho[gi(x, y + 1)]);
-                grho[i] += g[1][i] * (-0.5 * iy * iy);
-                grho[gi(x, y + 1)] += g[1][i] * (-0.5 * iy * iy);
-            } else {
-                grho[i] += g[1][i] * (-1.0 / (r * r));
-            }
-        }
-    const std::vector<double> &res = param == 0 ? gvp : (param == 1 ? gvs : grho);
-    std::memcpy(out, res.data(), n * sizeof(double));
+    if (s->model_h[0].size() != n) return fail(WV_ESTATE, "model not retained");
+    const double *c[5] = {a->grad[0], a->grad[1], a->grad[2], a->grad[3], a->grad[4]};
+    const float *m[3] = {s->model_h[0].data(), s->model_h[1].data(), s->model_h[2].data()};
+    HIP_TRY(wv::read_model_gradient(s->stage, 2, param, s->grid(), c, m, out, s->st));
     return WV_OK;
 }
 

@@ -456,93 +456,15 @@ int Elastic3D::get_gradient(int param, double *out)
     if (!a || !a->grad_ready) return fail(WV_ESTATE, "no gradient computed");
     if (param < 0 || param > 10 || !out) return fail(WV_EINVAL, "param must be 0..10");
     const size_t n = (size_t)NX * NY * NZ;
-    auto gi = [&](int x, int y, int z) { return (size_t)x + (size_t)z * NX + (size_t)y * NX * NZ; };
+    // coefficients (params 3..10) as they are; vp, vs, rho by the chain rule on the device (FP64)
     HIPA(hipStreamSynchronize(st));
-    std::vector<double> g[8];
-    std::vector<double> h((size_t)L.vol);
-    for (int k = 0; k < 8; k++) {
-        HIPA(hipMemcpy(h.data(), a->G.g[k], h.size() * 8, hipMemcpyDeviceToHost));
-        g[k].resize(n);
-        for (int y = 0; y < NY; y++)
-            for (int z = 0; z < NZ; z++)
-                for (int x = 0; x < NX; x++) g[k][gi(x, y, z)] = h[(size_t)L.at(x, y, z)];
-    }
     if (param >= 3) {
-        std::memcpy(out, g[param - 3].data(), n * 8);
+        HIPA(read_grid(stage, a->G.g[param - 3], grid(), out, st));
         return 0;
     }
-    // chain rule through the averaging rules (Modelparameter.cpp:336-639): coefficients -> vp, vs, rho
-    const std::vector<float> &vp = model_h[0], &vs = model_h[1], &rho = model_h[2];
-    if (vp.size() != n) return fail(WV_ESTATE, "model not retained");
-    std::vector<double> mu(n), gmu(g[4]), gvp(n, 0.0), gvs(n, 0.0), grho(n, 0.0);
-    for (size_t i = 0; i < n; i++) mu[i] = std::max((double)rho[i] * vs[i] * vs[i], 1.0);
-    const int len[3] = {NX, NY, NZ};
-    static const int planes[3][2] = {{0, 1}, {0, 2}, {1, 2}};
-    for (int pl = 0; pl < 3; pl++) {
-        const int a0 = planes[pl][0], a1 = planes[pl][1];
-        for (int y = 0; y < NY; y++)
-            for (int z = 0; z < NZ; z++)
-                for (int x = 0; x < NX; x++) {
-                    const int pos[3] = {x, y, z};
-                    const bool in0 = pos[a0] + 1 < len[a0], in1 = pos[a1] + 1 < len[a1];
-                    size_t pts[4];
-                    int np = 0;
-                    pts[np++] = gi(x, y, z);
-                    int p[3] = {x, y, z};
-                    if (in0) {
-                        p[a0]++;
-                        pts[np++] = gi(p[0], p[1], p[2]);
-                        p[a0]--;
-                    }
-                    if (in1) {
-                        p[a1]++;
-                        pts[np++] = gi(p[0], p[1], p[2]);
-                        p[a1]--;
-                    }
-                    if (in0 && in1) {
-                        p[a0]++;
-                        p[a1]++;
-                        pts[np++] = gi(p[0], p[1], p[2]);
-                    }
-                    const double w = 1.0 / np;
-                    double avg = 0;
-                    for (int q = 0; q < np; q++) avg += 1.0 / mu[pts[q]];
-                    const double m = 1.0 / (w * avg);
-                    if (m < 4.0) continue;  // the average is set to 0: no dependence
-                    const double gj = g[5 + pl][pts[0]];
-                    for (int q = 0; q < np; q++) gmu[pts[q]] += gj * m * m * w / (mu[pts[q]] * mu[pts[q]]);
-                }
-    }
-    for (size_t i = 0; i < n; i++) {
-        const double r = rho[i], p = vp[i], v = vs[i];
-        gvp[i] = g[3][i] * 2.0 * r * p;
-        grho[i] += g[3][i] * p * p;
-        if (r * v * v >= 1.0) {  // mu not clamped
-            gvs[i] = gmu[i] * 2.0 * r * v;
-            grho[i] += gmu[i] * v * v;
-        }
-    }
-    for (int ax = 0; ax < 3; ax++)
-        for (int y = 0; y < NY; y++)
-            for (int z = 0; z < NZ; z++)
-                for (int x = 0; x < NX; x++) {
-                    const int pos[3] = {x, y, z};
-                    const size_t i = gi(x, y, z);
-                    const double gk = g[ax][i];
-                    if (pos[ax] + 1 < len[ax]) {
-                        int p[3] = {x, y, z};
-                        p[ax]++;
-                        const size_t j = gi(p[0], p[1], p[2]);
-                        const double avg = 0.5 * ((double)rho[i] + rho[j]);
-                        const double d = -0.5 / (avg * avg);
-                        grho[i] += gk * d;
-                        grho[j] += gk * d;
-                    } else {
-                        grho[i] += gk * (-1.0 / ((double)rho[i] * rho[i]));
-                    }
-                }
-    const std::vector<double> &res = param == 0 ? gvp : (param == 1 ? gvs : grho);
-    std::memcpy(out, res.data(), n * 8);
+    if (model_h[0].size() != n) return fail(WV_ESTATE, "model not retained");
+    const float *m[3] = {model_h[0].data(), model_h[1].data(), model_h[2].data()};
+    HIPA(read_model_gradient(stage, 3, param, grid(), a->G.g, m, out, st));
     return 0;
 }
 

@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "../../include/wave_abi.h"
+#include "readback.hpp"
 #include "wave_internal.hpp"
 
 namespace wv {
@@ -159,6 +160,8 @@ class Elastic3D {
     struct Adj3State;
     Adj3State *adj3 = nullptr;
     std::vector<float> model_h[3];  // vp, vs, rho (chain rule of the gradient)
+    Staging stage;                  // results on their way to the host
+    PaddedGrid grid() const { return {L.NX, L.NY, L.NZ, L.at(0, 0, 0), L.slab, L.pitch}; }
     int run_segment(int t_start, int t_end, bool timed);
     int set_model_em(const float *m0, const float *m1, const float *m2);
     int psi_axis(int q) const;

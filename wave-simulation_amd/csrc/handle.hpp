@@ -11,6 +11,7 @@
 #include "../../include/wave_abi.h"
 #include "elastic3d.hpp"
 #include "plain.hpp"
+#include "readback.hpp"
 #include "wave_internal.hpp"
 
 // status + thread-local message returned through wv_last_error (abi.cpp)
@@ -116,6 +117,8 @@ struct wv_solver {
     // the model the gradient chain rule needs
     AdjointState *adj = nullptr;
     std::vector<float> model_h[3];
+    wv::Staging stage;    // results on their way to the host
+    wv::PaddedGrid grid() const { return {L.NX, L.NY, 1, L.at(0, 0), L.pitch, 0}; }
 
     // per-kernel timing (wv_set_kernel_timing)
     bool ktiming = false;

@@ -929,11 +929,7 @@ int Elastic3D::get_seismograms(int shot, float *out)
         return 0;
     }
     HIP3(hipStreamSynchronize(st));
-    std::vector<float> h((size_t)NT * rec_total);
-    HIP3(hipMemcpy(h.data(), d_seis, h.size() * sizeof(float), hipMemcpyDeviceToHost));
-    const int r0 = rec_ptr_h[shot];
-    for (int r = 0; r < nr; r++)
-        for (int t = 0; t < NT; t++) out[(size_t)r * NT + t] = h[(size_t)t * rec_total + r0 + r];
+    HIP3(read_traces(stage, d_seis, rec_total, rec_ptr_h[shot], nr, NT, out, st));
     return 0;
 }
 
@@ -946,17 +942,12 @@ void Elastic3D::buffers(wv::StateBuffers &out) const
 int Elastic3D::field_io(int shot, int field, float *out, const float *in)
 {
     if (field < 0 || field >= nf) return fail(WV_EINVAL, "bad field index");
-    std::vector<float> h((size_t)L.vol);
     float *d = F[field] + (size_t)shot * L.vol;
     HIP3(hipStreamSynchronize(st));
     if (out) {
-        HIP3(hipMemcpy(h.data(), d, h.size() * sizeof(float), hipMemcpyDeviceToHost));
-        for (int y = 0; y < NY; y++)
-            for (int z = 0; z < NZ; z++)
-                for (int x = 0; x < NX; x++)
-                    out[(size_t)x + (size_t)z * NX + (size_t)y * NX * NZ] = h[(size_t)L.at(x, y, z)];
+        HIP3(read_grid(stage, d, grid(), out, st));
     } else {
-        std::fill(h.begin(), h.end(), 0.f);
+        std::vector<float> h((size_t)L.vol, 0.f);
         for (int y = 0; y < NY; y++)
             for (int z = 0; z < NZ; z++)
                 for (int x = 0; x < NX; x++)

@@ -187,13 +187,13 @@ class ForwardSolver:
         names = self.GRADIENTS3D if self.dimension == "3D" else self.GRADIENTS
         k = names.index(param) if isinstance(param, str) else int(param)
         n = self.cfg.NX * self.cfg.NY * (self.cfg.NZ if self.dimension == "3D" else 1)
-        out = np.zeros(n, dtype=np.float64)
+        out = np.empty(n, dtype=np.float64)
         _abi.check(_abi.load().wv_get_gradient(self._h, k, out.ctypes.data_as(C.POINTER(C.c_double))))
         return out
 
     # -- results ------------------------------------------------------------------
     def seismograms(self, shot=0):
-        out = np.zeros((self._nrec.get(shot, 0), self.cfg.NT), dtype=np.float32)
+        out = np.empty((self._nrec.get(shot, 0), self.cfg.NT), dtype=np.float32)  # filled by the library
         if out.size:
             _abi.check(_abi.load().wv_get_seismograms(self._h, shot, _fp(out)))
         return out
@@ -202,7 +202,7 @@ class ForwardSolver:
         idx = name_or_index
         if isinstance(idx, str):
             idx = self.FIELDS[(self.dimension, self.type)].index(idx)
-        out = np.zeros(self.cfg.NX * self.cfg.NY * self.cfg.NZ, dtype=np.float32)
+        out = np.empty(self.cfg.NX * self.cfg.NY * self.cfg.NZ, dtype=np.float32)
         _abi.check(_abi.load().wv_get_wavefield(self._h, shot, idx, _fp(out)))
         return out
 
