@@ -15,84 +15,11 @@
 
 #include "buffer.hpp"
 #include "elastic3d.hpp"
+#include "tile3d.hpp"
 
 namespace wv {
 
 namespace {
-
-constexpr int NTH = TILE_X * BLOCK_Y;
-
-// Thread share of the region [x0-HX, x0+64+HX) x [z0-HZ, z0+TZ+HZ) of one y plane.
-template <int HX, int HZ, int TZ>
-struct Region {
-    static constexpr int RW = TILE_X + 2 * HX;
-    static constexpr int RH = TZ + 2 * HZ;
-    static constexpr int TOT = RW * RH;
-    static constexpr int IT = (TOT + NTH - 1) / NTH;
-    float v[IT];
-    __device__ __forceinline__ void load(const float *__restrict__ g, const Layout3D &L, int x0, int y, int z0, int tid)
-    {
-        const long long base = L.at(x0 - HX, y, z0 - HZ);
-#pragma unroll
-        for (int k = 0; k < IT; k++) {
-            const int i = tid + k * NTH;
-            if (TOT % NTH == 0 || i < TOT) {
-                const int r = i / RW;
-                const int c = i - r * RW;
-                v[k] = g[base + (long long)r * L.pitch + c];
-            }
-        }
-    }
-    __device__ __forceinline__ void store(float (*S)[RW], int tid) const
-    {
-#pragma unroll
-        for (int k = 0; k < IT; k++) {
-            const int i = tid + k * NTH;
-            if (TOT % NTH == 0 || i < TOT) {
-                const int r = i / RW;
-                const int c = i - r * RW;
-                S[r][c] = v[k];
-            }
-        }
-    }
-    // rows of an LDS array that every thread's share fits in (surplus threads write padding)
-    static constexpr int RHP = (IT * NTH + RW - 1) / RW;
-    // the same without a guard (S has RHP rows), so no divergent branch sits between the loads
-    // in flight and this store
-    __device__ __forceinline__ void store_padded(float (*S)[RW], int tid) const
-    {
-#pragma unroll
-        for (int k = 0; k < IT; k++) {
-            const int i = tid + k * NTH;
-            const int r = i / RW;
-            const int c = i - r * RW;
-            S[r][c] = v[k];
-        }
-    }
-};
-
-// Byte offsets, within one y plane, of a thread's share of a Region (the same
-// for every plane, so they are computed once per block).
-template <int HX, int HZ, int TZ>
-struct RegionOff {
-    using R = Region<HX, HZ, TZ>;
-    unsigned o[R::IT];
-    __device__ __forceinline__ void init(const Layout3D &L, int x0, int z0, int tid)
-    {
-#pragma unroll
-        for (int k = 0; k < R::IT; k++) {
-            const int i = min(tid + k * NTH, R::TOT - 1);  // surplus threads reload the last element
-            const int r = i / R::RW, c = i - r * R::RW;
-            o[k] = (unsigned)(((z0 - HZ + r + L.H) * L.pitch + (x0 - HX + c + XPAD)) * 4);
-        }
-    }
-};
-
-// One y plane of a field as a buffer resource (plane offsets stay 32-bit for any grid).
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t plane_rsrc(const float *f, const Layout3D &L, int y)
-{
-    return brsrc(f + (long long)(y + L.H) * L.slab, (unsigned)(L.slab * 4));
-}
 
 // Buffer offset that the hardware answers with 0 (loads) or drops (stores):
 // the CPML accesses of lanes outside a frame, without a branch.
@@ -169,15 +96,6 @@ struct ZTab {
 __device__ __forceinline__ bool tile_in_frame(const Layout3D &L, const Cpml3D &P, int x0, int z0, int TZ)
 {
     return P.on && (x0 < P.W || x0 + TILE_X > L.NX - P.W || z0 < P.W || z0 + TZ > L.NZ - P.W);
-}
-
-template <int HX, int HZ, int TZ>
-__device__ __forceinline__ void load_region(Region<HX, HZ, TZ> &g, const RegionOff<HX, HZ, TZ> &o, const float *f,
-                                            const Layout3D &L, int y)
-{
-    const auto b = plane_rsrc(f, L, y);
-#pragma unroll
-    for (int k = 0; k < Region<HX, HZ, TZ>::IT; k++) g.v[k] = bload(b, o.o[k], 0);
 }
 
 // derivative along x at LDS row r (array with an H-wide x halo), column tx
@@ -324,9 +242,17 @@ __device__ __forceinline__ Pos position(const Layout3D &L, int TZ, int nyc, int 
     return p;
 }
 
+// Wavefronts per SIMD the register allocation of the elastic kernels has to leave room for. With two
+// z rows per thread up to order 8 the kernels want 260 registers, 4 more than two wavefronts have: held
+// to 256 (at most 4 values go to scratch) two blocks share a CU and hide each other's loads, 2.85 ->
+// 2.08 ms per step for 4 shots of 256 x 200 x 240 at order 8. Orders 10 and 12 and the viscoelastic
+// stress would spill 28 to 106 registers inside the plane loop and keep one.
+constexpr int el3d_waves(int H, int RZ, bool VE = false) { return RZ == 2 && H <= 4 && !VE ? 2 : 1; }
+
 template <int H, int RZ, bool REC>
-__global__ __launch_bounds__(NTH) void el3d_velocity(Layout3D L, Fields3D F, Coef3D C, Taps3D T, Cpml3D P, Acq A,
-                                                     int nyc, int LY, int tofs, int pend, Rec3D R)
+__global__ __launch_bounds__(NTH, el3d_waves(H, RZ)) void el3d_velocity(Layout3D L, Fields3D F, Coef3D C, Taps3D T,
+                                                                       Cpml3D P, Acq A, int nyc, int LY, int tofs,
+                                                                       int pend, Rec3D R)
 {
     constexpr int TZ = RZ * BLOCK_Y, K = 2 * H + 1;
     using RX = Region<H, 0, TZ>;   // x derivatives only
@@ -669,8 +595,9 @@ __device__ __forceinline__ void ve3d_cell(const Visco3D &V, const Layout3D &L, l
 }
 
 template <int H, int RZ, bool REC, bool VE = false>
-__global__ __launch_bounds__(NTH) void el3d_stress(Layout3D L, Fields3D F, Coef3D C, Taps3D T, Cpml3D P, Acq A,
-                                                   int nyc, int LY, int tofs, Rec3D R, Visco3D V)
+__global__ __launch_bounds__(NTH, el3d_waves(H, RZ, VE)) void el3d_stress(Layout3D L, Fields3D F, Coef3D C, Taps3D T,
+                                                                         Cpml3D P, Acq A, int nyc, int LY, int tofs,
+                                                                         Rec3D R, Visco3D V)
 {
     constexpr int TZ = RZ * BLOCK_Y, K = 2 * H + 1;
     using RXZ = Region<H, H, TZ>;
