@@ -61,3 +61,26 @@ def test_depth_parts_are_never_empty():
                 planes = -(-NY // n)
                 assert (n - 1) * planes < NY <= n * planes, (NY, H, tiles, n)
                 assert planes == -(-NY // wanted)
+
+
+def test_depth_parts_fill_the_chip():
+    """wv::depth_parts_fill: the parts of depth_parts, or more of at least 2 planes, none empty, where
+    those leave part of the chip's block slots free; then no more blocks than slots."""
+    lib = ctypes.CDLL(abi.LIB_PATH)
+    f, g = lib["_ZN2wv11depth_partsEiiii"], lib["_ZN2wv16depth_parts_fillEiiiii"]
+    f.argtypes, f.restype = [ctypes.c_int] * 4, ctypes.c_int
+    g.argtypes, g.restype = [ctypes.c_int] * 5, ctypes.c_int
+    for H in range(1, 7):
+        for tiles in (1, 7, 40, 96, 480, 1500, 20000):
+            for slots in (256, 512, 1280):
+                for NY in range(2, 300):
+                    n, m = f(NY, H, tiles, 12288), g(NY, H, tiles, 12288, slots)
+                    planes = -(-NY // m)
+                    assert (m - 1) * planes < NY <= m * planes, (NY, H, tiles, slots, m)
+                    if m > n:
+                        assert m * tiles <= slots and planes >= 2
+                    elif m < n:
+                        raise AssertionError((NY, H, tiles, slots))
+                    elif n * tiles < slots:  # nothing more fits: one plane less per part is too many blocks
+                        p = -(-NY // n) - 1
+                        assert p < 2 or -(-NY // p) * tiles > slots

@@ -421,7 +421,8 @@ int Elastic3D::run_adjoint()
     const Cpml3D P = cpml();
     const Acq Q = acq();
     const TapsT3D TT{a->tapT[0], a->tapT[1], a->tapT[2], a->tapT[3], a->tapT[4], a->tapT[5]};
-    const int adj_nyc = nyc;  // parts of at least max(4H, 8) planes (depth_parts)
+    // the transposed stencils run with two rows per thread (two blocks per CU up to order 8)
+    const int adj_nyc = depth_parts_fill(NY, H, xz_tiles(2), kBlocks3D, kCus * (H <= 4 ? 2 : 1));
     for (int seg = a->nck - 1; seg >= 0; seg--) {
         const int s0 = seg * a->every, s1 = std::min(NT, s0 + a->every);
         if ((rc = restore_checkpoint(seg))) return rc;

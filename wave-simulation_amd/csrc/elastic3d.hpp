@@ -118,6 +118,12 @@ void launch_em3d(int which, int order, int rz, const Layout3D &L, int nshots, in
                  const Coef3D &C, const Taps3D &T, const Cpml3D &P, const Acq &A, int tofs, int pend,
                  hipStream_t stream, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr, const Visco3D *V = nullptr);
 
+// Blocks per launch the parts along depth aim at: about 48 per CU, so the last round of blocks
+// leaves little of the GPU idle (measured on 320^3 x 8 shots: 2048 -> 10.9 ms per step,
+// 12288 -> 10.1 ms; each part re-reads 2H planes).
+constexpr int kBlocks3D = 12288;
+constexpr int kCus = 256;         // compute units of the chip
+
 // Host driver of the 3D elastic solver (owned by a wv_solver handle).
 class Elastic3D {
   public:
@@ -212,6 +218,9 @@ class Elastic3D {
     int nps = 18;  // CPML memory variables (acoustic: p_x p_y p_z vx_x vy_y vz_z; EM: 12)
     double DT = 0, DH = 0, fc_ref = 0;  // fc_ref: CenterFrequencyCPML, the viscoelastic reference frequency
     int rz = 2, nyc = 1, nbx = 0, nbz = 0;
+    int xz_tiles(int r) const { return ((NX + TILE_X - 1) / TILE_X) * ((NZ + 4 * r - 1) / (4 * r)) * nshots; }
+    int blocks_per_cu(int r) const;
+    void split_depth();
     Layout3D L{};
     std::vector<void *> allocs, acq_allocs;
     float *F[9] = {};

@@ -227,4 +227,12 @@ std::vector<float> transpose_taps(const std::vector<float> &t, int H)
     return r;
 }
 
+int depth_parts_fill(int NY, int H, int tiles, int blocks, int slots)
+{
+    const int n = depth_parts(NY, H, tiles, blocks), m = std::min(slots / tiles, (NY + 1) / 2);
+    if (m <= n) return n;
+    const int planes = (NY + m - 1) / m;
+    return (NY + planes - 1) / planes;
+}
+
 }  // namespace wv

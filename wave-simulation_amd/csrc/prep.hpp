@@ -62,5 +62,8 @@ std::vector<double> abs_profile(int W, double damping_coeff);
 // each, and none of them empty (a block of a part beyond the grid would load its window of
 // planes from beyond the field).
 int depth_parts(int NY, int H, int tiles, int blocks);
+// The same for a chip that holds `slots` blocks at a time: where parts of that length leave it partly
+// idle, as many shorter ones (of at least 2 planes) as run at once.
+int depth_parts_fill(int NY, int H, int tiles, int blocks, int slots);
 
 }  // namespace wv

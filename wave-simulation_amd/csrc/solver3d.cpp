@@ -13,12 +13,6 @@
 
 namespace wv {
 
-// Blocks per launch the y chunking aims at: about 48 per CU, so the last round of blocks
-// leaves little of the GPU idle (measured on 320^3 x 8 shots: 2048 -> 10.9 ms per step,
-// 12288 -> 10.1 ms; each chunk re-reads 2H planes of y halo).
-constexpr int kBlocks3D = 12288;
-
-
 namespace {
 constexpr int ORG = 64;  // margin of position-indexed tables (see abi.cpp)
 int round_up(int v, int m) { return (v + m - 1) / m * m; }
@@ -136,7 +130,11 @@ int Elastic3D::init(const wv_config &k, hipStream_t stream, int phys, bool visco
     if (damping && 2 * W > std::min(NX, std::min(NY, NZ))) return fail(WV_EINVAL, "BoundaryWidth out of range");
     if (k.tile_y != 0 && k.tile_y != 4 && k.tile_y != 8 && k.tile_y != 16)
         return fail(WV_EINVAL, "tile_y of the 3D kernels must be 0 (default), 4, 8 or 16");
-    rz = k.tile_y ? k.tile_y / 4 : 2;
+    // Rows per thread before tuning: two read less halo, one makes twice the blocks, which is better
+    // while two leave the chip idle even in parts of 4 planes or hold one block
+    // per CU (us per step at order 8, two and one: 60^3 elastic 36 and 26, 64^3 acoustic 24 and 18, but
+    // 256 x 200 x 240 elastic 589 and 616; at order 12 961 and 685).
+    rz = k.tile_y ? k.tile_y / 4 : blocks_per_cu(2) < 2 || (long long)xz_tiles(2) * (NY / 4) < kCus * blocks_per_cu(2) ? 1 : 2;
 
     L.NX = NX;
     L.NY = NY;
@@ -264,9 +262,7 @@ int Elastic3D::init(const wv_config &k, hipStream_t stream, int phys, bool visco
         std::vector<int> zero(1, 0);
         if ((rc = upload(&d_tbase, zero, allocs))) return rc;
     }
-    // chunks along y: enough blocks to fill the chip, chunks of at least 4H planes
-    const int nxz = ((NX + TILE_X - 1) / TILE_X) * ((NZ + 4 * rz - 1) / (4 * rz)) * nshots;
-    nyc = depth_parts(NY, H, nxz, kBlocks3D);
+    split_depth();
     HIP3(hipEventCreate(&ev0));
     HIP3(hipEventCreate(&ev1));
     shots.assign(nshots, Shot());
@@ -274,11 +270,34 @@ int Elastic3D::init(const wv_config &k, hipStream_t stream, int phys, bool visco
     return 0;
 }
 
+// Blocks of the step's kernels that a CU holds at once with r z rows per thread (their registers;
+// the kernel that wants more of the two): elastic 2 (order 8, one row: 156 and 185 registers; two rows:
+// 256), above order 8 and viscoelastic 1 with two rows; acoustic 5 (95), with four rows 4 (128); EM 4 (102),
+// 3 (158) and 2 (252).
+int Elastic3D::blocks_per_cu(int r) const
+{
+    if (physics == ACOUSTIC) return r == 4 ? 4 : 5;
+    if (physics == TEMEM) return r == 1 ? 4 : r == 2 ? 3 : 2;
+    return r == 1 ? 2 : r == 2 && H <= 4 && !visco ? 2 : 1;
+}
+
+// Parts along depth. A block waits out one plane's loads after another, so its time goes with its
+// planes, and a grid too small to fill the chip with parts of 4H planes takes shorter ones: the planes
+// that a part reads before its first one (2H of three fields) come from the caches and cost less than
+// idle CUs. us per step untuned at order 8,
+// parts of 4H planes and now: elastic 96 x 72 x 80 of 2 shots 118 and 63, 128^3 111 and 88, 60^3 127 and 22,
+// acoustic 144 x 120 x 104 of 2 shots 115 and 74, 64^3 67 and 14, EM 100 x 90 x 80 161 and 39. Where the
+// chip is full either way, parts of 4H planes are as good or better (elastic 256 x 200 x 240: 584 to 662 for
+// parts of 4 to 32 planes, 589 with 16).
+void Elastic3D::split_depth()
+{
+    nyc = depth_parts_fill(NY, H, xz_tiles(rz), kBlocks3D, kCus * blocks_per_cu(rz));
+}
+
 int Elastic3D::set_rz(int r)
 {
     rz = r;
-    const int nxz = ((NX + TILE_X - 1) / TILE_X) * ((NZ + 4 * rz - 1) / (4 * rz)) * nshots;
-    nyc = depth_parts(NY, H, nxz, kBlocks3D);
+    split_depth();
     acq_dirty = true;
     drop_graph();
     return 0;
