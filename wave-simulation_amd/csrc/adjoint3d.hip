@@ -16,13 +16,11 @@
 // 4*RZ rows in LDS for the x and z terms, register queues of 2H+1 planes for the y
 // terms, marching along depth y.
 #include "adjoint3d.hpp"
-#include "buffer.hpp"
+#include "tile3d.hpp"
 
 namespace wv {
 
 namespace {
-
-constexpr int NTH = TILE_X * BLOCK_Y;
 
 // adjoint of the CPML update psi' = b psi + a d, d' = d + psi' for one cell:
 // given lh = adjoint of d', returns the adjoint of d and advances m (the adjoint of psi)
@@ -182,21 +180,23 @@ struct StencilMap<1> {
     static constexpr bool FWD[3][3] = {{true, false, false}, {false, true, false}, {false, false, true}};
 };
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t plane_res(const float *f, const Layout3D &L, int y)
-{
-    return brsrc(f + (long long)(y + L.H) * L.slab, (unsigned)(L.slab * 4));
-}
-
 // Transposed stencil phase: out[o] += sum over the terms of (D^T g).  Block = 64 x 4
 // threads over a 64-column x TZ-row x-z tile of one shot, marching over a chunk of y.
+// Everything the next plane reads is loaded while the current one is computed, at offsets
+// worked out once per block, and the barriers order LDS only, so a block waits for memory
+// once per plane and not between every load and its store: 96 x 72 x 80 cells of 2 shots
+// at order 8 134 and 140 us per launch before (in parts of 18 planes), 26 and 31 now (of 6).
 template <int H, int RZ, int PHASE>
-__global__ __launch_bounds__(NTH) void adj3d_stencil(Layout3D L, int nyc, Adj3D A, TapsT3D T)
+__global__ __launch_bounds__(NTH, H <= 4 ? 2 : 1) void adj3d_stencil(Layout3D L, int nyc, Adj3D A, TapsT3D T)
 {
     using M = StencilMap<PHASE>;
-    constexpr int TZ = RZ * BLOCK_Y, K = 2 * H + 1, RW = TILE_X + 2 * H, RH = TZ + 2 * H;
-    __shared__ float sx[3][TZ][RW];       // x terms with an x halo
-    __shared__ float sz[3][RH][TILE_X];   // z terms with a z halo
-    __shared__ float szt[2][TZ][K];       // z taps (transposed) of the tile's rows: [0] backward, [1] forward
+    constexpr int TZ = RZ * BLOCK_Y, K = 2 * H + 1;
+    using RX = Region<H, 0, TZ>;  // x terms: an x halo
+    using RZZ = Region<0, H, TZ>;  // z terms: a z halo
+    __shared__ float sx[3][RX::RHP][RX::RW];
+    __shared__ float sz[3][RZZ::RHP][RZZ::RW];
+    __shared__ float szt[2][TZ][K];  // z taps (transposed) of the tile's rows: [0] backward, [1] forward
+    __shared__ float syt[2][NTH];    // y taps (transposed) of the plane in [0, K): [0] backward, [1] forward
     const int nbx = gridDim.x;
     const int bx = blockIdx.x % nbx;
     const int bz = blockIdx.y;
@@ -204,7 +204,8 @@ __global__ __launch_bounds__(NTH) void adj3d_stencil(Layout3D L, int nyc, Adj3D 
     const int LY = (L.NY + nyc - 1) / nyc;
     const int ys = yc * LY, ye = min(L.NY, ys + LY);
     const int x0 = bx * TILE_X, z0 = bz * TZ;
-    const int tx = threadIdx.x, wz = threadIdx.y, tid = wz * TILE_X + tx;
+    const int tx = threadIdx.x, tid = threadIdx.y * TILE_X + tx;
+    const int wz = __builtin_amdgcn_readfirstlane(threadIdx.y);
     const int x = x0 + tx;
     const bool xin = x < L.NX;
     const long long so = (long long)shot * L.vol;
@@ -223,6 +224,10 @@ __global__ __launch_bounds__(NTH) void adj3d_stencil(Layout3D L, int nyc, Adj3D 
     unsigned oc[RZ];
 #pragma unroll
     for (int r = 0; r < RZ; r++) oc[r] = (unsigned)(((z0 + wz + r * BLOCK_Y + L.H) * L.pitch + x + XPAD) * 4);
+    RegionOff<H, 0, TZ> ox;
+    RegionOff<0, H, TZ> oz;
+    ox.init(L, x0, z0, tid);
+    oz.init(L, x0, z0, tid);
 
     // y queues of the three y terms, planes y-H .. y+H
     float q[3][K][RZ];
@@ -230,56 +235,55 @@ __global__ __launch_bounds__(NTH) void adj3d_stencil(Layout3D L, int nyc, Adj3D 
     for (int j = 0; j < 3; j++)
 #pragma unroll
         for (int k = 0; k < 2 * H; k++) {
-            const auto b = plane_res(A.g[3 + j] + so, L, ys - H + k);
+            const auto b = plane_rsrc(A.g[3 + j] + so, L, ys - H + k);
 #pragma unroll
             for (int r = 0; r < RZ; r++) q[j][k + 1][r] = bload(b, oc[r], 0);
         }
 
+    RX rx[3];
+    RZZ rz[3];
+    float nq[3][RZ], nxt[M::NOUT][RZ], ytb, ytf;
+    auto load_plane = [&](int y) {
+        ytb = T.yb[(long long)y * K + min(tid, K - 1)];
+        ytf = T.yf[(long long)y * K + min(tid, K - 1)];
+#pragma unroll
+        for (int j = 0; j < 3; j++) {
+            load_region(rx[j], ox, A.g[j] + so, L, y);
+            load_region(rz[j], oz, A.g[6 + j] + so, L, y);
+            const auto b = plane_rsrc(A.g[3 + j] + so, L, y + H);
+#pragma unroll
+            for (int r = 0; r < RZ; r++) nq[j][r] = bload(b, oc[r], 0);
+        }
+#pragma unroll
+        for (int o = 0; o < M::NOUT; o++) {
+            const auto b = plane_rsrc(A.l[M::OUT0 + o] + so, L, y);
+#pragma unroll
+            for (int r = 0; r < RZ; r++) nxt[o][r] = bload(b, oc[r], 0);
+        }
+    };
+    load_plane(ys);
+
     for (int y = ys; y < ye; y++) {
+        float acc[M::NOUT][RZ];
 #pragma unroll
         for (int j = 0; j < 3; j++) {
 #pragma unroll
             for (int k = 0; k < 2 * H; k++)
 #pragma unroll
                 for (int r = 0; r < RZ; r++) q[j][k][r] = q[j][k + 1][r];
-            const auto b = plane_res(A.g[3 + j] + so, L, y + H);
 #pragma unroll
-            for (int r = 0; r < RZ; r++) q[j][2 * H][r] = bload(b, oc[r], 0);
+            for (int r = 0; r < RZ; r++) q[j][2 * H][r] = nq[j][r];
+            rx[j].store_padded(sx[j], tid);
+            rz[j].store_padded(sz[j], tid);
         }
-        // x terms: rows z0 .. z0+TZ, columns x0-H .. x0+64+H
+        syt[0][tid] = ytb;  // (no guard: a divergent store here would wait for every load)
+        syt[1][tid] = ytf;
 #pragma unroll
-        for (int j = 0; j < 3; j++) {
-            const auto b = plane_res(A.g[j] + so, L, y);
-            for (int e = tid; e < TZ * RW; e += NTH) {
-                const int r = e / RW, c = e - r * RW;
-                sx[j][r][c] = bload(b, (unsigned)(((z0 + r + L.H) * L.pitch + x0 - H + c + XPAD) * 4), 0);
-            }
-        }
-        // z terms: rows z0-H .. z0+TZ+H, columns x0 .. x0+64
+        for (int o = 0; o < M::NOUT; o++)
 #pragma unroll
-        for (int j = 0; j < 3; j++) {
-            const auto b = plane_res(A.g[6 + j] + so, L, y);
-            for (int e = tid; e < RH * TILE_X; e += NTH) {
-                const int r = e / TILE_X, c = e - r * TILE_X;
-                sz[j][r][c] = bload(b, (unsigned)(((z0 - H + r + L.H) * L.pitch + x0 + c + XPAD) * 4), 0);
-            }
-        }
-        // outputs of this plane (read before the barrier, so the loads overlap it)
-        float acc[M::NOUT][RZ];
-#pragma unroll
-        for (int o = 0; o < M::NOUT; o++) {
-            const auto b = plane_res(A.l[M::OUT0 + o] + so, L, y);
-#pragma unroll
-            for (int r = 0; r < RZ; r++) acc[o][r] = bload(b, oc[r], 0);
-        }
-        // y taps (transposed) of this plane, the same for every lane
-        float cyf[K], cyb[K];
-#pragma unroll
-        for (int k = 0; k < K; k++) {
-            cyf[k] = T.yf[(long long)y * K + k];
-            cyb[k] = T.yb[(long long)y * K + k];
-        }
-        __syncthreads();
+            for (int r = 0; r < RZ; r++) acc[o][r] = nxt[o][r];
+        block_sync_lds();
+        load_plane(min(y + 1, ye - 1));  // (the last plane again: no branch between the loads and their use)
 #pragma unroll
         for (int r = 0; r < RZ; r++) {
             const int lz = wz + r * BLOCK_Y;
@@ -289,7 +293,7 @@ __global__ __launch_bounds__(NTH) void adj3d_stencil(Layout3D L, int nyc, Adj3D 
 #pragma unroll
                 for (int k = 0; k < K; k++) {
                     sxv += (M::FWD[0][j] ? cxf[k] : cxb[k]) * sx[j][lz][tx + k];
-                    syv += (M::FWD[1][j] ? cyf[k] : cyb[k]) * q[j][k][r];
+                    syv += syt[M::FWD[1][j] ? 1 : 0][k] * q[j][k][r];
                     szv += szt[M::FWD[2][j] ? 1 : 0][lz][k] * sz[j][lz + k][tx];
                 }
                 acc[M::OUT[0][j]][r] += sxv;
@@ -302,9 +306,9 @@ __global__ __launch_bounds__(NTH) void adj3d_stencil(Layout3D L, int nyc, Adj3D 
             const int z = z0 + wz + r * BLOCK_Y;
             if (!xin || z >= L.NZ) continue;
 #pragma unroll
-            for (int o = 0; o < M::NOUT; o++) bstore(acc[o][r], plane_res(A.l[M::OUT0 + o] + so, L, y), oc[r], 0);
+            for (int o = 0; o < M::NOUT; o++) bstore(acc[o][r], plane_rsrc(A.l[M::OUT0 + o] + so, L, y), oc[r], 0);
         }
-        __syncthreads();  // the next plane rewrites the LDS tiles
+        block_sync_lds();  // the next plane rewrites the LDS tiles
     }
 }
 
