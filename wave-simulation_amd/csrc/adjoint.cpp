@@ -15,7 +15,7 @@
 // checkpoints nor recomputation.
 // Gradients with respect to 1/rho_x, 1/rho_y, M, mu, mu_xy accumulate in FP64
 // on the GPU; the chain rule to vp, vs, rho follows the averaging rules of the
-// coefficient preparation (host, FP64).
+// coefficient preparation (FP64, readback.hip).
 #include <cmath>
 #include <cstring>
 
