@@ -240,8 +240,8 @@ int wv_set_checkpointing(wv_solver *s, int every, int fp16);
 /* Device-memory budget [GiB] for recording, during the checkpointed forward
  * run, the five derivative sums of every step (FP16, one scale per row of 64
  * cells, field and shot: about 10 B per cell, shot and step) instead of
- * checkpointing and recomputing; used when the handle runs the row-strip
- * kernels and the record fits.  < 0 (default): 3/4 of the free device memory
+ * checkpointing and recomputing; used when the handle was given the row-strip
+ * kernels, by WV_PATH_STRIP or by wv_tune, and the record fits.  < 0 (default): 3/4 of the free device memory
  * at wv_set_checkpointing; 0: always checkpoint and recompute.  Takes effect
  * at the next wv_set_checkpointing.  No counterpart in the reference. */
 int wv_set_adjoint_store(wv_solver *s, double max_gib);

@@ -89,6 +89,18 @@ def test_gradient_matches_fp64_oracle(fp16):
         assert e <= GTOL, (name, e)
 
 
+@pytest.mark.parametrize("fp16", [False, True])
+def test_default_handle_checkpoints_and_recomputes(fp16):
+    """A handle that names neither path nor tile height keeps the checkpoints it was asked for, and recomputes in
+    FP32: with the default record budget its gradient is the two-launch handle's (whose kernels have no record) up
+    to the order of the FP64 atomics.  The FP16 record moves it by about 1e-5."""
+    c, obs = _c4(N=130, NT=200)
+    _, ga, _, _ = _gpu_gradient(c, obs, every=40, fp16=fp16, store=-1.0)
+    _, gb, _, _ = _gpu_gradient(c, obs, every=40, fp16=fp16, store=-1.0, path="phased", tile_y=16)
+    for k, name in enumerate(("vp", "vs", "rho")):
+        assert rel_l2(ga[k], gb[k]) <= 1e-12, (name, rel_l2(ga[k], gb[k]))
+
+
 @pytest.mark.parametrize("tile_y", [8, 16])
 def test_gradient_with_row_strip_recomputation(tile_y):
     """The recomputation runs on the row-strip kernels (they record the derivative sums too)."""

@@ -458,6 +458,7 @@ int wv_init(wv_solver *s, const wv_config *c)
         // which is faster than the single-pass kernel at every size measured (C2: 20.5 against
         // 38.3 us per step)
         s->variant = V_STRIP;
+        s->strip_default = true;
         s->tile_x = wv::TILE_X;
         s->tile_y = 16;
     }
@@ -1257,6 +1258,7 @@ int wv_tune(wv_solver *s, int nsteps, int *choice)
         }
     }
     s->variant = cand_var[best_k];
+    s->strip_default = false;
     s->tile_x = s->variant == V_SINGLE ? wv::fused2d_tile_x(s->cfg.spatial_fd_order) : wv::TILE_X;
     s->tile_y = cand_ty[best_k];
     s->acq_dirty = true;
@@ -1268,6 +1270,7 @@ int wv_tune(wv_solver *s, int nsteps, int *choice)
         const int v0 = s->variant, tx0 = s->tile_x, ty0 = s->tile_y;
         if (s->physics == wv::ELASTIC && s->variant != V_STRIP && wv::strip2d_fits(s->L)) {
             s->variant = V_STRIP;
+            s->strip_default = true;
             s->tile_x = wv::TILE_X;
             s->tile_y = 16;
         }
@@ -1291,6 +1294,7 @@ int wv_tune(wv_solver *s, int nsteps, int *choice)
             if (choice) *choice = 13;
         } else {
             s->variant = v0;
+            s->strip_default = false;
             s->tile_x = tx0;
             s->tile_y = ty0;
         }

@@ -9,8 +9,8 @@
 // the gradient needs (the five CPML-modified derivative sums), then runs the
 // adjoint steps of the segment in reverse order.
 // When the FP16 record of every step of the run fits in the device-memory
-// budget (wv_set_adjoint_store) and the handle runs the row-strip kernels,
-// the forward run records the sums of every step directly (FP16, one scale
+// budget (wv_set_adjoint_store) and the handle was given the row-strip kernels
+// by its path or by wv_tune, the forward run records the sums of every step directly (FP16, one scale
 // per row of 64 cells, field and shot) and the backward pass needs neither
 // checkpoints nor recomputation.
 // Gradients with respect to 1/rho_x, 1/rho_y, M, mu, mu_xy accumulate in FP64
@@ -273,8 +273,9 @@ int wv_set_checkpointing(wv_solver *s, int every, int fp16)
     a->fld_n = (size_t)s->L.plane * s->cfg.nshots;
     a->nck = (s->cfg.NT + every - 1) / every;
     a->have.assign(a->nck, 0);
-    // record every step instead when it fits (row-strip kernels only)
-    if (s->variant == V_STRIP) {
+    // record every step instead when it fits (row-strip kernels only, and only where the caller or
+    // wv_tune chose them: the record is FP16, and a handle that runs them by default recomputes in FP32)
+    if (s->variant == V_STRIP && !s->strip_default) {
         const int nbx = (s->L.NX + wv::TILE_X - 1) / wv::TILE_X, srows = s->tile_y / 4;
         const int nty = (s->L.NY + srows - 1) / srows;
         const size_t fss = (size_t)s->cfg.NT * 5 * s->cfg.nshots;  // (step, field, shot) planes

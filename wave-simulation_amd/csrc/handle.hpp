@@ -57,6 +57,8 @@ struct wv_solver {
 
     int variant = V_PHASED;
     int tile_x = wv::TILE_X, tile_y = wv::TILE_Y;  // tiling of the kernels in use
+    // the row-strip kernels are the handle's default, neither named by its path nor measured by wv_tune
+    bool strip_default = false;
     int tile_load = 1;  // single-pass kernel: -1 direct global->LDS loads, 1 register-staged loads
     wv::Layout2D L{};
     int H = 0;
