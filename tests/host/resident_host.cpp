@@ -1,0 +1,183 @@
+// The resident loop's host side (resident2d.cpp) over a stand-in for the HIP runtime: memory comes from
+// malloc and can be made to run out at a chosen allocation, and launches are noted instead of run.
+//   resident_host <test> [number]
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <set>
+#include <string>
+#include <vector>
+
+#include "handle.hpp"
+#include "resident2d.hpp"
+
+#define CHECK(c)                                                                \
+    do {                                                                        \
+        if (!(c)) {                                                             \
+            std::fprintf(stderr, "line %d: not true: %s\n", __LINE__, #c);      \
+            std::exit(1);                                                       \
+        }                                                                       \
+    } while (0)
+
+namespace {
+
+std::set<void *> live;
+int allocations = 0, fail_at = 0;  // the fail_at-th allocation finds no memory (0: none)
+int launches = 0;
+std::string last_error;
+
+hipError_t give(void **p, size_t n)
+{
+    if (++allocations == fail_at) return hipErrorOutOfMemory;
+    *p = std::calloc(1, n ? n : 1);
+    live.insert(*p);
+    return hipSuccess;
+}
+hipError_t take(void *p)
+{
+    CHECK(!p || live.erase(p) == 1);
+    std::free(p);
+    return hipSuccess;
+}
+
+hipError_t launch(const wv::ResGo &g)
+{
+    if (g.capacity) {
+        *g.capacity = 256;
+        return hipSuccess;
+    }
+    const wv::Res2DArgs &X = *g.X;
+    CHECK(X.xch && X.ctl && X.host && X.bsrc_ptr && X.bsrc && X.brec_ptr && X.brec);
+    CHECK(X.psi || !g.P->on);
+    launches++;
+    X.host[0] = 2 * X.launch;
+    return hipSuccess;
+}
+
+}  // namespace
+
+int wv_fail(int code, const std::string &msg)
+{
+    last_error = msg;
+    return code;
+}
+wv_solver::~wv_solver()
+{
+    res2d_destroy(this);
+    free_list(allocs);
+}
+
+namespace wv {
+hipError_t res2d_el(int, bool, const void *go) { return launch(*(const ResGo *)go); }
+hipError_t res2d_ac(int, bool, const void *go) { return launch(*(const ResGo *)go); }
+hipError_t res2d_tm(int, bool, const void *go) { return launch(*(const ResGo *)go); }
+hipError_t res2d_sh(int, bool, const void *go) { return launch(*(const ResGo *)go); }
+}  // namespace wv
+
+extern "C" {
+hipError_t hipMalloc(void **p, size_t n) { return give(p, n); }
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return give(p, n); }
+hipError_t hipFree(void *p) { return take(p); }
+hipError_t hipHostFree(void *p) { return take(p); }
+hipError_t hipMemsetAsync(void *p, int v, size_t n, hipStream_t)
+{
+    std::memset(p, v, n);
+    return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t)
+{
+    std::memcpy(d, s, n);
+    return hipSuccess;
+}
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamQuery(hipStream_t) { return hipSuccess; }
+hipError_t hipGetDevice(int *d)
+{
+    *d = 0;
+    return hipSuccess;
+}
+hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t, int)
+{
+    *v = 256;
+    return hipSuccess;
+}
+hipError_t hipGetLastError() { return hipSuccess; }
+const char *hipGetErrorString(hipError_t) { return "error"; }
+hipError_t hipEventCreate(hipEvent_t *e)
+{
+    *e = nullptr;
+    return hipSuccess;
+}
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t)
+{
+    *ms = 1.f;
+    return hipSuccess;
+}
+}
+
+namespace {
+
+void make(wv_solver &s)
+{
+    s.physics = wv::ELASTIC;
+    s.cfg.NX = s.L.NX = 200;
+    s.cfg.NY = s.L.NY = 150;
+    s.cfg.NZ = 1;
+    s.cfg.NT = 1000;
+    s.cfg.spatial_fd_order = 8;
+    s.H = 4;
+    s.cfg.damping_boundary = 2;
+    s.cfg.nshots = 2;
+    s.variant = V_STRIP;
+    s.tile_y = 16;
+    s.inited = s.model_ok = true;
+    s.shots.resize(2);
+    for (ShotAcq &a : s.shots) {
+        a.sidx = {75 * 200 + 100};
+        a.ridx = {10 * 200 + 30, 140 * 200 + 190};
+    }
+}
+
+// Whichever allocation fails, nothing is kept of the others, no launch is made with a part of the buffers,
+// and the caller is told to run the steps with the ordinary kernels, now and the next time.
+void no_memory()
+{
+    int total = 0;
+    {
+        wv_solver s;
+        make(s);
+        CHECK(res2d_run(&s, 0, 100) == 0 && launches == 1);
+        total = allocations;
+    }
+    CHECK(live.empty());
+    CHECK(total == 8);  // exchange words, control words, memory variables, report words, four lists
+    for (int k = 1; k <= total; k++) {
+        allocations = launches = 0;
+        fail_at = k;
+        {
+            wv_solver s;
+            make(s);
+            CHECK(res2d_run(&s, 0, 100) == 1);
+            CHECK(live.size() <= 1);  // (the report words stay with the handle)
+            CHECK(res2d_run(&s, 100, 200) == 1);
+            CHECK(launches == 0);
+        }
+        CHECK(live.empty());
+    }
+}
+
+}  // namespace
+
+int main(int argc, char **argv)
+{
+    const std::string t = argc > 1 ? argv[1] : "";
+    if (t == "no_memory")
+        no_memory();
+    else
+        CHECK(!"a known test");
+    std::puts("ok");
+    return 0;
+}

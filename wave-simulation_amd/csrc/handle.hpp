@@ -137,8 +137,8 @@ struct wv_solver {
         void *q = nullptr;
         if (n == 0) n = 1;
         if (hipMalloc(&q, n * sizeof(T)) != hipSuccess) return fail(WV_ENOMEM, "hipMalloc failed");
-        if (hipMemsetAsync(q, 0, n * sizeof(T), st) != hipSuccess) return fail(WV_EDEVICE, "hipMemset failed");
         list.push_back(q);
+        if (hipMemsetAsync(q, 0, n * sizeof(T), st) != hipSuccess) return fail(WV_EDEVICE, "hipMemset failed");
         *p = (T *)q;
         return 0;
     }

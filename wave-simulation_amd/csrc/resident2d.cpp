@@ -5,7 +5,7 @@
 #include <algorithm>
 
 #include "handle.hpp"
-#include "resident2d_launch.hpp"
+#include "resident2d.hpp"
 
 namespace wv {
 
@@ -216,6 +216,79 @@ static bool res_plan(wv_solver *s, int srow)
     return (bool)r->plan;
 }
 
+// The plan's exchange buffer, control words, memory variables and report words: all of them or none.
+// False: a handle whose device memory is used up keeps the ordinary kernels, which need none of these.
+static bool res_buffers(wv_solver *s)
+{
+    Res2DState *r = s->res;
+    if (r->xch) return true;
+    const wv::Res2DPlan &p = r->plan;
+    int phase1 = 0;
+    const size_t words = wv::res2d_words(s->physics, s->H, p.rows(), &phase1);
+    const size_t npsi = (size_t)p.blocks() * p.nwv * 4 * (s->physics == wv::ELASTIC ? 2 : 1) * p.srow * 64;
+    std::vector<void *> got;
+    unsigned long long *xch = nullptr;
+    unsigned *ctl = nullptr;
+    float *psi = nullptr;
+    if (s->dalloc(&xch, words * p.blocks(), got) || s->dalloc(&ctl, 3, got) ||
+        (s->cfg.damping_boundary == 2 && s->dalloc(&psi, npsi, got)) ||
+        (!r->host && hipHostMalloc((void **)&r->host, 64, hipHostMallocDefault) != hipSuccess)) {
+        (void)hipGetLastError();
+        s->free_list(got);
+        return false;
+    }
+    r->host[0] = r->host[1] = 0;
+    r->allocs = got;
+    r->words = (int)words;
+    r->phase1 = phase1;
+    r->ctl = ctl;
+    r->psi = psi;
+    r->xch = xch;
+    return true;
+}
+
+// The acquisition per (shot, tile of the plan): all four lists or none.
+static bool res_lists(wv_solver *s)
+{
+    Res2DState *r = s->res;
+    if (r->lists) return true;
+    const wv::Res2DPlan &p = r->plan;
+    const int R = p.rows();
+    const size_t nsb = (size_t)s->cfg.nshots * p.nby * p.nbx;
+    std::vector<std::vector<int>> bs(nsb), br(nsb);
+    int gs = 0, gr = 0;
+    for (int sh = 0; sh < s->cfg.nshots; sh++) {
+        auto blk = [&](long long g) {
+            const int x = (int)(g % s->L.NX), y = (int)(g / s->L.NX);
+            return ((size_t)sh * p.nby + y / R) * p.nbx + x / wv::TILE_X;
+        };
+        for (long long g : s->shots[sh].sidx) bs[blk(g)].push_back(gs++);
+        for (long long g : s->shots[sh].ridx) br[blk(g)].push_back(gr++);
+    }
+    std::vector<int> bsp(1, 0), bsl, brp(1, 0), brl;
+    for (size_t b = 0; b < nsb; b++) {
+        bsl.insert(bsl.end(), bs[b].begin(), bs[b].end());
+        bsp.push_back((int)bsl.size());
+        brl.insert(brl.end(), br[b].begin(), br[b].end());
+        brp.push_back((int)brl.size());
+    }
+    std::vector<void *> got;
+    int *q[4] = {};
+    if (s->upload(&q[0], bsp, got) || s->upload(&q[1], bsl, got) || s->upload(&q[2], brp, got) ||
+        s->upload(&q[3], brl, got)) {
+        (void)hipGetLastError();
+        s->free_list(got);
+        return false;
+    }
+    r->acq_allocs = got;
+    r->bsrc_ptr = q[0];
+    r->bsrc = q[1];
+    r->brec_ptr = q[2];
+    r->brec = q[3];
+    r->lists = true;
+    return true;
+}
+
 // nsteps steps from t0 in one launch.  0: done (enqueued and started); 1: not started (the caller
 // runs the steps with the ordinary kernels); < 0: error.
 int res2d_run(wv_solver *s, int t0, int nsteps, const wv::Rec2D *rec, float *snap, long long snap_field,
@@ -224,41 +297,12 @@ int res2d_run(wv_solver *s, int t0, int nsteps, const wv::Rec2D *rec, float *sna
     if (!res_plan(s, rec || snap ? s->tile_y / 4 : 0)) return 1;
     Res2DState *r = s->res;
     const wv::Res2DPlan &p = r->plan;
-    int rc;
-    if (!r->xch) {
-        r->words = (int)wv::res2d_words(s->physics, s->H, p.rows(), &r->phase1);
-        if ((rc = s->dalloc(&r->xch, (size_t)r->words * p.blocks(), r->allocs)) || (rc = s->dalloc(&r->ctl, 3, r->allocs)) ||
-            (s->cfg.damping_boundary == 2 &&
-             (rc = s->dalloc(&r->psi, (size_t)p.blocks() * p.nwv * 4 * (s->physics == wv::ELASTIC ? 2 : 1) * p.srow * 64,
-                             r->allocs))))
-            return rc;
-        if (!r->host) HIP_TRY(hipHostMalloc((void **)&r->host, 64, hipHostMallocDefault));
-        r->host[0] = r->host[1] = 0;
-    }
-    if (!r->lists) {
-        const int R = p.rows();
-        const size_t nsb = (size_t)s->cfg.nshots * p.nby * p.nbx;
-        std::vector<std::vector<int>> bs(nsb), br(nsb);
-        int gs = 0, gr = 0;
-        for (int sh = 0; sh < s->cfg.nshots; sh++) {
-            auto blk = [&](long long g) {
-                const int x = (int)(g % s->L.NX), y = (int)(g / s->L.NX);
-                return ((size_t)sh * p.nby + y / R) * p.nbx + x / wv::TILE_X;
-            };
-            for (long long g : s->shots[sh].sidx) bs[blk(g)].push_back(gs++);
-            for (long long g : s->shots[sh].ridx) br[blk(g)].push_back(gr++);
-        }
-        std::vector<int> bsp(1, 0), bsl, brp(1, 0), brl;
-        for (size_t b = 0; b < nsb; b++) {
-            bsl.insert(bsl.end(), bs[b].begin(), bs[b].end());
-            bsp.push_back((int)bsl.size());
-            brl.insert(brl.end(), br[b].begin(), br[b].end());
-            brp.push_back((int)brl.size());
-        }
-        if ((rc = s->upload(&r->bsrc_ptr, bsp, r->acq_allocs)) || (rc = s->upload(&r->bsrc, bsl, r->acq_allocs)) ||
-            (rc = s->upload(&r->brec_ptr, brp, r->acq_allocs)) || (rc = s->upload(&r->brec, brl, r->acq_allocs)))
-            return rc;
-        r->lists = true;
+    if (!res_buffers(s) || !res_lists(s)) {
+        // no memory: this handle stays with the ordinary kernels from here on
+        s->free_list(r->allocs);
+        r->xch = nullptr;
+        r->plan = wv::Res2DPlan{};
+        return 1;
     }
     wv::Res2DArgs X{};
     X.nwv = p.nwv;

@@ -46,6 +46,22 @@ struct Res2DKernArgs {
     Rec2D R;
 };
 
+// What a per-physics launcher (resident2d_*.hip) is asked for.
+struct ResGo {
+    const Res2DPlan *plan;
+    const Layout2D *L;
+    const Fields2D *F;
+    const Coef2D *C;
+    const Taps *T;
+    const Cpml2D *P;
+    const Acq *A;
+    const Res2DArgs *X;
+    Rec2D rec;
+    hipStream_t st;
+    int *capacity;  // not null: report the blocks resident at once instead of launching
+    size_t lds;
+};
+
 // The plan the estimate prefers (empty: none fits); *gain = estimated step time of the two-launch
 // kernels over the plan's.
 Res2DPlan res2d_plan(int physics, int order, const Layout2D &L, int nshots, int srow, double *gain);

@@ -8,21 +8,6 @@
 namespace wv {
 namespace {
 
-struct ResGo {
-    const Res2DPlan *plan;
-    const Layout2D *L;
-    const Fields2D *F;
-    const Coef2D *C;
-    const Taps *T;
-    const Cpml2D *P;
-    const Acq *A;
-    const Res2DArgs *X;
-    Rec2D rec;
-    hipStream_t st;
-    int *capacity;  // not null: report the blocks resident at once instead of launching
-    size_t lds;
-};
-
 template <typename Kern>
 hipError_t res_launch(Kern k, const ResGo &g)
 {
