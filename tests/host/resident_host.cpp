@@ -1,6 +1,6 @@
 // The resident loop's host side (resident2d.cpp) over a stand-in for the HIP runtime: memory comes from
 // malloc and can be made to run out at a chosen allocation, and launches are noted instead of run.
-//   resident_host <test> [number]
+//   resident_host <test>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -22,6 +22,7 @@
 namespace {
 
 std::set<void *> live;
+size_t live_bytes = 0;
 int allocations = 0, fail_at = 0;  // the fail_at-th allocation finds no memory (0: none)
 int launches = 0;
 std::string last_error;
@@ -31,6 +32,7 @@ hipError_t give(void **p, size_t n)
     if (++allocations == fail_at) return hipErrorOutOfMemory;
     *p = std::calloc(1, n ? n : 1);
     live.insert(*p);
+    live_bytes += n;
     return hipSuccess;
 }
 hipError_t take(void *p)
@@ -169,6 +171,28 @@ void no_memory()
     }
 }
 
+// A memory plan is told at least what the loop's buffers take, before they are there.
+void memory_asked_for()
+{
+    for (int physics : {wv::ELASTIC, wv::ACOUSTIC, wv::TMEM, wv::SH})
+        for (int damping = 0; damping < 3; damping++) {
+            live_bytes = 0;
+            wv_solver s;
+            make(s);
+            s.physics = physics;
+            s.cfg.damping_boundary = damping;
+            const size_t said = res2d_bytes(&s, 0);
+            CHECK(live_bytes == 0);
+            CHECK(res2d_run(&s, 0, 100) == 0);
+            const size_t words = 64 + 3 * sizeof(unsigned);  // report and control words
+            CHECK(said >= live_bytes - words && said <= live_bytes);
+        }
+    wv_solver s;
+    make(s);
+    s.visco = true;
+    CHECK(res2d_bytes(&s, 0) == 0);
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
@@ -176,6 +200,8 @@ int main(int argc, char **argv)
     const std::string t = argc > 1 ? argv[1] : "";
     if (t == "no_memory")
         no_memory();
+    else if (t == "memory_asked_for")
+        memory_asked_for();
     else
         CHECK(!"a known test");
     std::puts("ok");

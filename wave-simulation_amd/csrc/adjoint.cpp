@@ -283,11 +283,13 @@ int wv_set_checkpointing(wv_solver *s, int every, int fp16)
         const double need = (double)words * 4 + (double)strips * 4;
         size_t free_b = 0, total_b = 0;
         HIP_TRY(hipMemGetInfo(&free_b, &total_b));
-        // what wv_run_adjoint allocates later must still fit next to the record: the five
-        // adjoint fields, two sets of CPML memory variables, the FP64 gradient planes, the
-        // transposed tap tables and the time-major adjoint sources
+        // what is allocated later must still fit next to the record: the five adjoint fields, two
+        // sets of CPML memory variables, the FP64 gradient planes, the transposed tap tables and the
+        // time-major adjoint sources (wv_run_adjoint), the resident loop's buffers, the staging of
+        // the read-backs
         const double later = (double)a->fld_n * 5 * 4 + 2.0 * (double)psi_total(s) * 4 +
-                             (double)s->L.plane * 5 * 8 + (double)s->cfg.NT * (s->rec_total + 1) * 4 + 64.0e6;
+                             (double)s->L.plane * 5 * 8 + (double)s->cfg.NT * (s->rec_total + 1) * 4 + 64.0e6 +
+                             (double)res2d_bytes(s, srows) + (double)wv::Staging::kStageBytes;
         const double avail = std::max(0.0, (double)free_b - later);
         const double budget = a->store_gib < 0 ? 0.75 * avail : std::min(a->store_gib * 1073741824.0, avail);
         if (need <= budget) {

@@ -311,6 +311,7 @@ void res2d_acquisition_changed(wv_solver *s);
 bool res2d_eligible(const wv_solver *s);
 int res2d_run(wv_solver *s, int t0, int nsteps, const wv::Rec2D *rec = nullptr, float *snap = nullptr,
               long long snap_field = 0, long long snap_step = 0);
+size_t res2d_bytes(wv_solver *s, int srow);  // device bytes its buffers will want
 bool res2d_expected(wv_solver *s, bool rec);
 bool res2d_failed(const wv_solver *s);
 extern const char *const kResidentFailed;

@@ -216,6 +216,29 @@ static bool res_plan(wv_solver *s, int srow)
     return (bool)r->plan;
 }
 
+// Floats of a plan's memory variables.
+static size_t res_psi(const wv_solver *s, const wv::Res2DPlan &p)
+{
+    if (s->cfg.damping_boundary != 2) return 0;
+    return (size_t)p.blocks() * p.nwv * 4 * (s->physics == wv::ELASTIC ? 2 : 1) * p.srow * wv::TILE_X;
+}
+
+// Device bytes that runs of the handle with that many rows per wavefront (0: the planner's choice) will
+// want for the loop, for memory plans that divide what is free.
+size_t res2d_bytes(wv_solver *s, int srow)
+{
+    if (!res2d_eligible(s)) return 0;
+    double gain = 0.0;
+    const wv::Res2DPlan p = wv::res2d_plan(s->physics, s->cfg.spatial_fd_order, s->L, s->cfg.nshots, srow, &gain);
+    if (!p) return 0;
+    int phase1 = 0;
+    size_t n = wv::res2d_words(s->physics, s->H, p.rows(), &phase1) * p.blocks() * sizeof(unsigned long long);
+    n += res_psi(s, p) * sizeof(float);
+    size_t ids = 2 * (size_t)s->cfg.nshots * p.nby * p.nbx + 2;
+    for (const ShotAcq &a : s->shots) ids += a.sidx.size() + a.ridx.size();
+    return n + ids * sizeof(int);
+}
+
 // The plan's exchange buffer, control words, memory variables and report words: all of them or none.
 // False: a handle whose device memory is used up keeps the ordinary kernels, which need none of these.
 static bool res_buffers(wv_solver *s)
@@ -225,13 +248,13 @@ static bool res_buffers(wv_solver *s)
     const wv::Res2DPlan &p = r->plan;
     int phase1 = 0;
     const size_t words = wv::res2d_words(s->physics, s->H, p.rows(), &phase1);
-    const size_t npsi = (size_t)p.blocks() * p.nwv * 4 * (s->physics == wv::ELASTIC ? 2 : 1) * p.srow * 64;
+    const size_t npsi = res_psi(s, p);
     std::vector<void *> got;
     unsigned long long *xch = nullptr;
     unsigned *ctl = nullptr;
     float *psi = nullptr;
     if (s->dalloc(&xch, words * p.blocks(), got) || s->dalloc(&ctl, 3, got) ||
-        (s->cfg.damping_boundary == 2 && s->dalloc(&psi, npsi, got)) ||
+        (npsi && s->dalloc(&psi, npsi, got)) ||
         (!r->host && hipHostMalloc((void **)&r->host, 64, hipHostMallocDefault) != hipSuccess)) {
         (void)hipGetLastError();
         s->free_list(got);
