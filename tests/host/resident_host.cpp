@@ -1,4 +1,4 @@
-// The resident loop's host side (resident2d.cpp) over a stand-in for the HIP runtime: memory comes from
+// The resident loop's host side (resident2d.cpp) and the read-backs' staging (readback.hpp) over a stand-in for the HIP runtime: memory comes from
 // malloc and can be made to run out at a chosen allocation, and launches are noted instead of run.
 //   resident_host <test>
 #include <cstdio>
@@ -24,7 +24,8 @@ namespace {
 std::set<void *> live;
 size_t live_bytes = 0;
 int allocations = 0, fail_at = 0;  // the fail_at-th allocation finds no memory (0: none)
-int launches = 0;
+size_t device_left = ~(size_t)0;   // largest device allocation that is still to be had
+int launches = 0, copies = 0;
 std::string last_error;
 
 hipError_t give(void **p, size_t n)
@@ -77,7 +78,7 @@ hipError_t res2d_sh(int, bool, const void *go) { return launch(*(const ResGo *)g
 }  // namespace wv
 
 extern "C" {
-hipError_t hipMalloc(void **p, size_t n) { return give(p, n); }
+hipError_t hipMalloc(void **p, size_t n) { return n > device_left ? hipErrorOutOfMemory : give(p, n); }
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return give(p, n); }
 hipError_t hipFree(void *p) { return take(p); }
 hipError_t hipHostFree(void *p) { return take(p); }
@@ -88,6 +89,7 @@ hipError_t hipMemsetAsync(void *p, int v, size_t n, hipStream_t)
 }
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t)
 {
+    copies++;
     std::memcpy(d, s, n);
     return hipSuccess;
 }
@@ -193,6 +195,43 @@ void memory_asked_for()
     CHECK(res2d_bytes(&s, 0) == 0);
 }
 
+// Read-backs take what device memory there is, down to one item, then pinned host memory.
+void staging()
+{
+    const size_t M = 1u << 20;
+    {
+        wv::Staging S;
+        CHECK(S.reserve(100, M, 0) == 64);  // cut to the limit
+        CHECK(S.reserve(10, M, 0) == 10 && live.size() == 1);
+    }
+    CHECK(live.empty());
+    device_left = 20 * M;
+    {
+        wv::Staging S;
+        CHECK(S.reserve(100, M, 0) == 16);
+        CHECK(S.reserve(2, 3 * M, M) == 2);
+    }
+    device_left = 0;
+    {
+        wv::Staging S;
+        CHECK(S.reserve(100, 3 * sizeof(int), sizeof(int)) == 1);
+        CHECK(live.size() == 1);
+        const int in[3] = {1, 2, 3};
+        int out[3] = {};
+        CHECK(S.copy_in(S.data(), in, sizeof(in), nullptr) == hipSuccess);
+        CHECK(S.copy_out(out, S.data(), sizeof(out), nullptr) == hipSuccess);
+        CHECK(out[0] == 1 && out[2] == 3 && copies == 0);  // (host memory: no device copy)
+        device_left = 1000;
+        CHECK(S.reserve(10, 12, 4) == 10);  // device memory again
+        CHECK(S.copy_out(out, S.data(), sizeof(out), nullptr) == hipSuccess && copies == 1);
+    }
+    CHECK(live.empty());
+    fail_at = allocations + 1;
+    wv::Staging S;
+    device_left = 0;
+    CHECK(S.reserve(1, 8, 0) == 0);
+}
+
 }  // namespace
 
 int main(int argc, char **argv)
@@ -202,6 +241,8 @@ int main(int argc, char **argv)
         no_memory();
     else if (t == "memory_asked_for")
         memory_asked_for();
+    else if (t == "staging")
+        staging();
     else
         CHECK(!"a known test");
     std::puts("ok");

@@ -1,5 +1,5 @@
-"""Host side of the resident 2D time loop, without a GPU: resident2d.cpp compiled against a stand-in for the
-HIP runtime (tests/host/resident_host.cpp)."""
+"""Host side of the resident 2D time loop, without a GPU: resident2d.cpp and the read-backs' staging
+compiled against a stand-in for the HIP runtime (tests/host/resident_host.cpp)."""
 import os
 import subprocess
 
@@ -18,7 +18,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("test", ["no_memory", "memory_asked_for"])
+@pytest.mark.parametrize("test", ["no_memory", "memory_asked_for", "staging"])
 def test_resident_host(program, test):
     r = subprocess.run([program, test], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout.strip() == "ok", r.stderr

@@ -9,8 +9,6 @@
 // 96 x 72 x 80 cells 37 -> 0.54 ms.
 #include "readback.hpp"
 
-#include <algorithm>
-
 namespace wv {
 
 namespace {
@@ -135,30 +133,12 @@ hipError_t read_rows(Staging &S, const T *f, const PaddedGrid &g, T *out, hipStr
         const size_t ny = std::min(part, g.NY - y), n = ny * g.row();
         pack<T><<<blocks(n), 256, 0, st>>>(f, g, (int)y, (int)ny, d);
         TRY(hipGetLastError());
-        TRY(hipMemcpyAsync(out + y * g.row(), d, n * sizeof(T), hipMemcpyDeviceToHost, st));
+        TRY(S.copy_out(out + y * g.row(), d, n * sizeof(T), st));
     }
     return hipStreamSynchronize(st);
 }
 
 }  // namespace
-
-size_t Staging::reserve(size_t items, size_t bytes, size_t extra)
-{
-    items = std::min(items, std::max<size_t>(1, (kStageBytes - std::min(kStageBytes, extra)) / bytes));
-    for (; items; items /= 2) {
-        const size_t need = items * bytes + extra;
-        if (need <= n_) return items;
-        if (p_) (void)hipFree(p_);
-        n_ = 0;
-        if (hipMalloc((void **)&p_, need) == hipSuccess) {
-            n_ = need;
-            return items;
-        }
-        (void)hipGetLastError();
-        p_ = nullptr;
-    }
-    return 0;
-}
 
 hipError_t read_traces(Staging &S, const float *seis, int total, int r0, int nr, int NT, float *out, hipStream_t st)
 {
@@ -171,7 +151,7 @@ hipError_t read_traces(Staging &S, const float *seis, int total, int r0, int nr,
         const int n = (int)std::min(part, nr - r);
         traces<<<dim3((NT + 63) / 64, (n + 63) / 64), 256, 0, st>>>(seis, total, r0 + (int)r, n, NT, d);
         TRY(hipGetLastError());
-        TRY(hipMemcpyAsync(out + r * NT, d, (size_t)n * NT * sizeof(float), hipMemcpyDeviceToHost, st));
+        TRY(S.copy_out(out + r * NT, d, (size_t)n * NT * sizeof(float), st));
     }
     return hipStreamSynchronize(st);
 }
@@ -203,14 +183,14 @@ hipError_t read_model_gradient(Staging &S, int dim, int param, const PaddedGrid 
         const size_t ya = y ? y - 1 : 0, yb = std::min<size_t>(g.NY, y + ny + 1), n = (yb - ya) * row;
         for (int k = 0; k < 3; k++) {
             *m[k] = md + k * (part + 2) * row;
-            TRY(hipMemcpyAsync((void *)*m[k], model[k] + ya * row, n * sizeof(float), hipMemcpyHostToDevice, st));
+            TRY(S.copy_in((void *)*m[k], model[k] + ya * row, n * sizeof(float), st));
         }
         if (dim == 2)
             chain_rule<2><<<blocks(ny * row), 256, 0, st>>>(param, g, (int)y, (int)ny, A, d);
         else
             chain_rule<3><<<blocks(ny * row), 256, 0, st>>>(param, g, (int)y, (int)ny, A, d);
         TRY(hipGetLastError());
-        TRY(hipMemcpyAsync(out + y * row, d, ny * row * sizeof(double), hipMemcpyDeviceToHost, st));
+        TRY(S.copy_out(out + y * row, d, ny * row * sizeof(double), st));
     }
     return hipStreamSynchronize(st);
 }
