@@ -26,6 +26,7 @@ size_t live_bytes = 0;
 int allocations = 0, fail_at = 0;  // the fail_at-th allocation finds no memory (0: none)
 size_t device_left = ~(size_t)0;   // largest device allocation that is still to be had
 int launches = 0, copies = 0;
+bool refuse = false;  // not all blocks of a launch come in
 std::string last_error;
 
 hipError_t give(void **p, size_t n)
@@ -53,7 +54,7 @@ hipError_t launch(const wv::ResGo &g)
     CHECK(X.xch && X.ctl && X.host && X.bsrc_ptr && X.bsrc && X.brec_ptr && X.brec);
     CHECK(X.psi || !g.P->on);
     launches++;
-    X.host[0] = 2 * X.launch;
+    X.host[0] = 2 * X.launch + refuse;
     return hipSuccess;
 }
 
@@ -195,6 +196,25 @@ void memory_asked_for()
     CHECK(res2d_bytes(&s, 0) == 0);
 }
 
+// Only a launch that ran is reported as the timed kernel.
+void timing()
+{
+    wv_solver s;
+    make(s);
+    s.ktiming = true;
+    refuse = true;
+    CHECK(res2d_run(&s, 0, 100) == 1 && launches == 1);
+    CHECK(!res2d_timed(&s) && s.klaunch[0] == 0);
+    refuse = false;
+    wv_solver t;
+    make(t);
+    t.ktiming = true;
+    CHECK(res2d_run(&t, 0, 100) == 0);
+    CHECK(res2d_timed(&t) && t.klaunch[0] == 100);
+    res2d_timing_reset(&t);
+    CHECK(!res2d_timed(&t));
+}
+
 // Read-backs take what device memory there is, down to one item, then pinned host memory.
 void staging()
 {
@@ -241,6 +261,8 @@ int main(int argc, char **argv)
         no_memory();
     else if (t == "memory_asked_for")
         memory_asked_for();
+    else if (t == "timing")
+        timing();
     else if (t == "staging")
         staging();
     else

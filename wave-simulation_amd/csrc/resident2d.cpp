@@ -358,7 +358,6 @@ int res2d_run(wv_solver *s, int t0, int nsteps, const wv::Rec2D *rec, float *sna
             if (!ev) HIP_TRY(hipEventCreate(&ev));
         e0 = r->ev[0];
         e1 = r->ev[1];
-        r->timed = true;
         HIP_TRY(hipEventRecord(e0, s->st));
     }
     const hipError_t e = wv::launch_res2d(s->physics, s->cfg.spatial_fd_order, p, s->L, s->fields2d(s->cur), s->coef2d(),
@@ -392,6 +391,7 @@ int res2d_run(wv_solver *s, int t0, int nsteps, const wv::Rec2D *rec, float *sna
             HIP_TRY(hipEventElapsedTime(&ms, e0, e1));
             s->kms[0] += ms;
             s->klaunch[0] += nsteps;  // counted per time step
+            r->timed = true;
         }
         return 0;
     }
