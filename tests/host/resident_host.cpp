@@ -27,6 +27,8 @@ int allocations = 0, fail_at = 0;  // the fail_at-th allocation finds no memory 
 size_t device_left = ~(size_t)0;   // largest device allocation that is still to be had
 int launches = 0, copies = 0;
 bool refuse = false;  // not all blocks of a launch come in
+bool give_up = false;  // a launch's wait runs out
+wv::Res2DArgs last;    // arguments of the last launch
 std::string last_error;
 
 hipError_t give(void **p, size_t n)
@@ -54,7 +56,12 @@ hipError_t launch(const wv::ResGo &g)
     CHECK(X.xch && X.ctl && X.host && X.bsrc_ptr && X.bsrc && X.brec_ptr && X.brec);
     CHECK(X.psi || !g.P->on);
     launches++;
+    last = X;
     X.host[0] = 2 * X.launch + refuse;
+    if (give_up && !refuse) {
+        X.ctl[2] = 1;
+        X.host[1] = X.launch;
+    }
     return hipSuccess;
 }
 
@@ -216,6 +223,66 @@ void timing()
     CHECK(!res2d_timed(&t));
 }
 
+// A wait that ran out is reported until wv_reset, through plans given up and made, and not afterwards.
+void failure()
+{
+    wv_solver s;
+    make(s);
+    const wv::Rec2D rec{};
+    CHECK(!res2d_failed(&s));
+    CHECK(res2d_run(&s, 0, 100) == 0 && !res2d_failed(&s));
+    give_up = true;
+    CHECK(res2d_run(&s, 100, 100) == 0 && res2d_failed(&s));
+    give_up = false;
+    CHECK(res2d_run(&s, 0, 100, &rec) == 0);  // another plan, another set of buffers
+    CHECK(res2d_failed(&s));
+    CHECK(res2d_run(&s, 0, 100) == 0);
+    CHECK(res2d_failed(&s));
+    last.ctl[2] = 1;
+    CHECK(res2d_reset(&s) == 0);
+    CHECK(!res2d_failed(&s) && last.ctl[2] == 0);
+    CHECK(res2d_run(&s, 0, 100) == 0 && !res2d_failed(&s));
+    // a launch from before the reset may still be at it
+    const unsigned before = last.launch;
+    CHECK(res2d_reset(&s) == 0);
+    last.host[1] = before;
+    CHECK(!res2d_failed(&s));
+    give_up = true;
+    CHECK(res2d_run(&s, 0, 100) == 0 && res2d_failed(&s));
+}
+
+// A refused check-in leaves the steps to the ordinary kernels until wv_reset, three in a row for good.
+void refusal()
+{
+    wv_solver s;
+    make(s);
+    const wv::Rec2D rec{};
+    refuse = true;
+    for (int k = 1; k <= 3; k++) {
+        CHECK(res2d_run(&s, 0, 100) == 1 && launches == k);
+        CHECK(res2d_run(&s, 100, 100) == 1 && res2d_run(&s, 200, 100, &rec) == 1 && launches == k);
+        CHECK(res2d_reset(&s) == 0);
+    }
+    CHECK(res2d_run(&s, 0, 100) == 1 && launches == 3);
+    wv_solver t;
+    make(t);
+    launches = 0;
+    for (int k = 1; k <= 4; k++) {  // not in a row
+        refuse = true;
+        CHECK(res2d_run(&t, 0, 100) == 1);
+        CHECK(res2d_reset(&t) == 0);
+        refuse = false;
+        CHECK(res2d_run(&t, 0, 100) == 0 && launches == 2 * k);
+    }
+    // the same for want of memory
+    wv_solver u;
+    make(u);
+    fail_at = allocations + 2;
+    CHECK(res2d_run(&u, 0, 100) == 1 && res2d_run(&u, 0, 100) == 1);
+    CHECK(res2d_reset(&u) == 0);
+    CHECK(res2d_run(&u, 0, 100) == 0);
+}
+
 // Read-backs take what device memory there is, down to one item, then pinned host memory.
 void staging()
 {
@@ -264,6 +331,10 @@ int main(int argc, char **argv)
         memory_asked_for();
     else if (t == "timing")
         timing();
+    else if (t == "failure")
+        failure();
+    else if (t == "refusal")
+        refusal();
     else if (t == "staging")
         staging();
     else

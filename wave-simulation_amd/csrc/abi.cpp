@@ -303,7 +303,7 @@ double wv_solver::kernel_bytes(int kind) const
 }
 
 const char *const kResidentFailed =
-    "the resident time loop gave up waiting for its halos: the run's fields and seismograms are not valid";
+    "the resident time loop gave up waiting for its halos: fields and seismograms are not valid until wv_reset";
 
 extern "C" {
 
@@ -1020,7 +1020,7 @@ int wv_reset(wv_solver *s)
     if (s->d_seis) HIP_TRY(hipMemsetAsync(s->d_seis, 0, (size_t)s->cfg.NT * std::max(s->rec_total, 1) * 4, s->st));
     for (int k = 0; k < 12; k++)
         if (s->vR[k]) HIP_TRY(hipMemsetAsync(s->vR[k], 0, fn * sizeof(float), s->st));
-    return WV_OK;
+    return res2d_reset(s);
 }
 
 // Shorter run segments stay with the two-launch kernels: a resident launch costs its set-up and one pass
@@ -1048,6 +1048,7 @@ int wv_run(wv_solver *s, int t_start, int t_end)
         s->ran = true;
         return WV_OK;
     }
+    if (res2d_failed(s)) return fail(WV_EDEVICE, kResidentFailed);
     int rc = s->sync_acquisition();
     if (rc) return rc;
     HIP_TRY(hipEventRecord(s->ev0, s->st));

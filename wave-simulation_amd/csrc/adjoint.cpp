@@ -372,6 +372,7 @@ int wv_run_adjoint(wv_solver *s)
     }
     if (!s || !s->inited || !s->adj || !s->adj->every) return fail(WV_ESTATE, "checkpointing is not enabled");
     AdjointState *a = s->adj;
+    if (res2d_failed(s)) return fail(WV_EDEVICE, kResidentFailed);
     if (!a->forward_done) return fail(WV_ESTATE, "wv_run_adjoint needs a checkpointed forward run over [0, NT)");
     for (int k = 0; k < a->nck; k++)
         if (!a->have[k]) return fail(WV_ESTATE, "missing checkpoint");

@@ -314,6 +314,7 @@ int res2d_run(wv_solver *s, int t0, int nsteps, const wv::Rec2D *rec = nullptr, 
 size_t res2d_bytes(wv_solver *s, int srow);  // device bytes its buffers will want
 bool res2d_expected(wv_solver *s, bool rec);
 bool res2d_failed(const wv_solver *s);
+int res2d_reset(wv_solver *s);
 extern const char *const kResidentFailed;
 bool res2d_timed(const wv_solver *s);  // the timed run calls went through the resident loop
 void res2d_timing_reset(wv_solver *s);

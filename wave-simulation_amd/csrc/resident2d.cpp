@@ -162,9 +162,13 @@ struct Res2DState {
     unsigned long long *xch = nullptr;
     unsigned *ctl = nullptr;
     float *psi = nullptr;
-    unsigned *host = nullptr;  // pinned
+    unsigned *host = nullptr;  // pinned, one for the handle's life: see Res2DArgs
     int words = 0, phase1 = 0;  // exchange words of a block
-    unsigned tag = 1, arrived = 0, launches = 0;
+    unsigned tag = 1, arrived = 0;
+    unsigned launches = 0;  // made in the handle's life
+    unsigned first = 1;     // the first one since the last wv_reset
+    bool off = false;       // the ordinary kernels run the steps until the next wv_reset
+    int refused = 0;        // check-ins refused in a row
     hipEvent_t ev[2] = {};  // per-kernel timing
     bool timed = false;     // the timed run calls went through the resident loop
 };
@@ -202,6 +206,7 @@ static bool res_plan(wv_solver *s, int srow)
 {
     if (!s->res) s->res = new Res2DState();
     Res2DState *r = s->res;
+    if (r->off) return false;
     if (r->planned && r->srow == srow) return (bool)r->plan;
     s->free_list(r->acq_allocs);
     s->free_list(r->allocs);
@@ -212,7 +217,7 @@ static bool res_plan(wv_solver *s, int srow)
     r->xch = nullptr;
     r->ctl = nullptr;
     r->tag = 1;
-    r->arrived = r->launches = 0;
+    r->arrived = 0;
     return (bool)r->plan;
 }
 
@@ -253,14 +258,18 @@ static bool res_buffers(wv_solver *s)
     unsigned long long *xch = nullptr;
     unsigned *ctl = nullptr;
     float *psi = nullptr;
+    unsigned *host = nullptr;
     if (s->dalloc(&xch, words * p.blocks(), got) || s->dalloc(&ctl, 3, got) ||
         (npsi && s->dalloc(&psi, npsi, got)) ||
-        (!r->host && hipHostMalloc((void **)&r->host, 64, hipHostMallocDefault) != hipSuccess)) {
+        (!r->host && hipHostMalloc((void **)&host, 64, hipHostMallocDefault) != hipSuccess)) {
         (void)hipGetLastError();
         s->free_list(got);
         return false;
     }
-    r->host[0] = r->host[1] = 0;
+    if (host) {
+        host[0] = host[1] = 0;
+        r->host = host;
+    }
     r->allocs = got;
     r->words = (int)words;
     r->phase1 = phase1;
@@ -321,10 +330,11 @@ int res2d_run(wv_solver *s, int t0, int nsteps, const wv::Rec2D *rec, float *sna
     Res2DState *r = s->res;
     const wv::Res2DPlan &p = r->plan;
     if (!res_buffers(s) || !res_lists(s)) {
-        // no memory: this handle stays with the ordinary kernels from here on
+        // no memory
         s->free_list(r->allocs);
         r->xch = nullptr;
-        r->plan = wv::Res2DPlan{};
+        r->planned = false;
+        r->off = true;
         return 1;
     }
     wv::Res2DArgs X{};
@@ -384,6 +394,7 @@ int res2d_run(wv_solver *s, int t0, int nsteps, const wv::Rec2D *rec, float *sna
         sched_yield();
     }
     if (h[0] == go) {
+        r->refused = 0;
         if (e0) {
             HIP_TRY(hipEventRecord(e1, s->st));
             HIP_TRY(hipEventSynchronize(e1));
@@ -395,16 +406,37 @@ int res2d_run(wv_solver *s, int t0, int nsteps, const wv::Rec2D *rec, float *sna
         }
         return 0;
     }
-    // something else holds the GPU: this handle stays with the ordinary kernels from here on
-    r->plan = wv::Res2DPlan{};
+    // something else holds the GPU
+    r->off = true;
+    r->refused++;
     return 1;
 }
 
 // Whether the planner expects the resident loop to be the faster one for the handle's run calls.
 bool res2d_expected(wv_solver *s, bool rec) { return res_plan(s, rec ? s->tile_y / 4 : 0) && s->res->gain > 1.05; }
 
-// A wait inside a resident launch ran out (checked where results are handed out).
-bool res2d_failed(const wv_solver *s) { return s->res && s->res->host && ((volatile unsigned *)s->res->host)[1]; }
+// A wait inside a resident launch ran out: the state is not valid until wv_reset. (Every call that would go
+// on from the state or hand it out asks here first. The report names the launch, so it outlives the buffers
+// of a plan, and one from before the reset does not count.)
+bool res2d_failed(const wv_solver *s)
+{
+    if (!s->res || !s->res->host) return false;
+    const unsigned launch = ((volatile unsigned *)s->res->host)[1];
+    return launch && (int)(launch - s->res->first) >= 0;
+}
+
+// wv_reset: what went wrong before does not matter any more, in stream order. The loop is tried again after
+// a refused check-in (one other kernel may have been the cause, and a refusal costs 0.3 s), but not after
+// three of them in a row.
+int res2d_reset(wv_solver *s)
+{
+    Res2DState *r = s->res;
+    if (!r) return 0;
+    r->first = r->launches + 1;
+    if (r->refused < 3) r->off = false;
+    if (r->xch) HIP_TRY(hipMemsetAsync(r->ctl + 2, 0, sizeof(unsigned), s->st));
+    return 0;
+}
 
 bool res2d_timed(const wv_solver *s) { return s->res && s->res->timed; }
 void res2d_timing_reset(wv_solver *s)

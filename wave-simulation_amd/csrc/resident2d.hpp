@@ -26,7 +26,7 @@ struct Res2DArgs {
     unsigned tag0;             // tag of the launch's first step
     unsigned *ctl;             // [0] blocks arrived (all launches), [1] verdict, [2] a wait ran out
     unsigned arrive, launch;   // value of ctl[0] when all blocks of this launch are in; launch number
-    volatile unsigned *host;   // pinned: [0] verdict of the launch, [1] a wait ran out
+    volatile unsigned *host;   // pinned: [0] verdict of the launch, [1] the launch whose wait ran out last
     const int *bsrc_ptr, *bsrc, *brec_ptr, *brec;  // acquisition lists per (shot, tile) of this plan
     float *psi;                // memory variables of the resident tiles, [block][wavefront][psi_wave floats]
     float *snap;               // elastic: segment record (Snap2D planes of step t0), or nullptr

@@ -721,7 +721,7 @@ __global__ __launch_bounds__(MAXT, MINW) void res2d(Res2DKernArgs KA)
         if (bad) {
             if (tid == 0) {
                 __hip_atomic_store(KA.X.ctl + 2, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(const_cast<unsigned *>(KA.X.host) + 1, 1u, __ATOMIC_RELAXED,
+                __hip_atomic_store(const_cast<unsigned *>(KA.X.host) + 1, KA.X.launch, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_SYSTEM);
             }
             return;
