@@ -139,9 +139,14 @@ int wv_set_acquisition(wv_solver *s, int shot, int nsrc, const long long *src_in
  * shape with a window (2, 3, 5, 6) shifted beyond the signal, with the reference's messages. */
 int wv_source_signal(int shape, int NT, double DT, double fc, double amp, double tshift, float *out);
 
+/* zero wavefields, CPML memory variables and seismograms; also what a handle needs after WV_EDEVICE for a
+ * resident loop that gave up waiting (wv_run and the read-backs report it until then) */
 int wv_reset(wv_solver *s);
 
-/* advance all shots over time steps [t_start, t_end); asynchronous on the handle's stream */
+/* advance all shots over time steps [t_start, t_end); asynchronous on the handle's stream.  A resident
+ * launch that does not find the GPU to itself within 0.3 s (other kernels hold part of it) leaves its
+ * steps undone; the next call that waits for the handle, or that needs its state or acquisition as they
+ * are, has the ordinary kernels run them, and those of the calls queued behind it, in order. */
 int wv_run(wv_solver *s, int t_start, int t_end);
 int wv_synchronize(wv_solver *s);
 

@@ -1,9 +1,11 @@
 // The resident loop's host side (resident2d.cpp) and the read-backs' staging (readback.hpp) over a stand-in for the HIP runtime: memory comes from
-// malloc and can be made to run out at a chosen allocation, and launches are noted instead of run.
+// malloc and can be made to run out at a chosen allocation; launches and copies go to a stream that works
+// when it is waited for, or told to, and notes what was run.
 //   resident_host <test>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <set>
 #include <string>
 #include <vector>
@@ -46,22 +48,52 @@ hipError_t take(void *p)
     return hipSuccess;
 }
 
+// The stream: what is queued, and a note of what was run ("R" resident, "O" ordinary steps, "C" a checkpoint).
+std::vector<std::function<void()>> stream;
+std::string ran;
+void work(size_t n)
+{
+    for (size_t k = 0; k < n && k < stream.size(); k++) stream[k]();
+    stream.erase(stream.begin(), stream.begin() + std::min(n, stream.size()));
+}
+void note(const char *what, int t0, int n)
+{
+    ran += std::string(what) + std::to_string(t0) + (n ? "+" + std::to_string(n) : "") + " ";
+}
+std::string take_notes()
+{
+    std::string s;
+    s.swap(ran);
+    return s;
+}
+
 hipError_t launch(const wv::ResGo &g)
 {
     if (g.capacity) {
         *g.capacity = 256;
         return hipSuccess;
     }
-    const wv::Res2DArgs &X = *g.X;
+    const wv::Res2DArgs X = *g.X;
     CHECK(X.xch && X.ctl && X.host && X.bsrc_ptr && X.bsrc && X.brec_ptr && X.brec);
     CHECK(X.psi || !g.P->on);
     launches++;
     last = X;
-    X.host[0] = 2 * X.launch + refuse;
-    if (give_up && !refuse) {
-        X.ctl[2] = 1;
-        X.host[1] = X.launch;
-    }
+    // the check-in of resident2d_kernel.hpp, all blocks at once
+    stream.push_back([X] {
+        CHECK(live.count(X.ctl) && live.count(X.xch) && live.count((void *)X.brec));
+        X.ctl[0] += X.nbx * X.nby * X.conc;
+        CHECK(X.ctl[0] == X.arrive);
+        const unsigned behind = X.ctl[3];
+        const bool stop = behind || refuse;
+        if (stop) X.ctl[3] = behind ? behind : X.launch;
+        X.host[0] = stop ? ((unsigned long long)X.ctl[3] << 32) | (2 * X.launch + 1) : 2 * X.launch;
+        if (stop) return;
+        note("R", X.t0, X.nsteps);
+        if (give_up) {
+            X.ctl[2] = 1;
+            X.host[1] = X.launch;
+        }
+    });
     return hipSuccess;
 }
 
@@ -74,11 +106,26 @@ int wv_fail(int code, const std::string &msg)
 }
 wv_solver::~wv_solver()
 {
+    (void)hipStreamSynchronize(nullptr);
     res2d_destroy(this);
     free_list(allocs);
 }
 
+int step_base = 0;
+int wv_solver::enqueue_steps(int n, bool)
+{
+    const int t0 = step_base;
+    stream.push_back([t0, n] { note("O", t0, n); });
+    return 0;
+}
+int adjoint_checkpoint_again(wv_solver *, int t)
+{
+    stream.push_back([t] { note("C", t, 0); });
+    return 0;
+}
+
 namespace wv {
+void launch_set(int *, int v, hipStream_t) { step_base = v; }
 hipError_t res2d_el(int, bool, const void *go) { return launch(*(const ResGo *)go); }
 hipError_t res2d_ac(int, bool, const void *go) { return launch(*(const ResGo *)go); }
 hipError_t res2d_tm(int, bool, const void *go) { return launch(*(const ResGo *)go); }
@@ -88,21 +135,29 @@ hipError_t res2d_sh(int, bool, const void *go) { return launch(*(const ResGo *)g
 extern "C" {
 hipError_t hipMalloc(void **p, size_t n) { return n > device_left ? hipErrorOutOfMemory : give(p, n); }
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return give(p, n); }
-hipError_t hipFree(void *p) { return take(p); }
+hipError_t hipFree(void *p)
+{
+    work(stream.size());  // (hipFree waits for the device)
+    return take(p);
+}
 hipError_t hipHostFree(void *p) { return take(p); }
 hipError_t hipMemsetAsync(void *p, int v, size_t n, hipStream_t)
 {
-    std::memset(p, v, n);
+    stream.push_back([p, v, n] { std::memset(p, v, n); });
     return hipSuccess;
 }
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t)
 {
     copies++;
+    work(stream.size());  // (pageable memory)
     std::memcpy(d, s, n);
     return hipSuccess;
 }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
-hipError_t hipStreamQuery(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t)
+{
+    work(stream.size());
+    return hipSuccess;
+}
 hipError_t hipGetDevice(int *d)
 {
     *d = 0;
@@ -123,7 +178,7 @@ hipError_t hipEventCreate(hipEvent_t *e)
 }
 hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
-hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipStreamSynchronize(nullptr); }
 hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t)
 {
     *ms = 1.f;
@@ -195,7 +250,7 @@ void memory_asked_for()
             const size_t said = res2d_bytes(&s, 0);
             CHECK(live_bytes == 0);
             CHECK(res2d_run(&s, 0, 100) == 0);
-            const size_t words = 64 + 3 * sizeof(unsigned);  // report and control words
+            const size_t words = 64 + 4 * sizeof(unsigned);  // report and control words
             CHECK(said >= live_bytes - words && said <= live_bytes);
         }
     wv_solver s;
@@ -212,7 +267,7 @@ void timing()
     s.ktiming = true;
     refuse = true;
     CHECK(res2d_run(&s, 0, 100) == 1 && launches == 1);
-    CHECK(!res2d_timed(&s) && s.klaunch[0] == 0);
+    CHECK(!res2d_timed(&s) && s.klaunch[0] == 0 && take_notes().empty());
     refuse = false;
     wv_solver t;
     make(t);
@@ -223,6 +278,13 @@ void timing()
     CHECK(!res2d_timed(&t));
 }
 
+// 0 / 1: the steps went through the loop / the ordinary kernels
+int run(wv_solver &s, int t0, int n, const wv::Rec2D *rec = nullptr)
+{
+    const int rc = res2d_run(&s, t0, n, rec);
+    return rc ? rc : res2d_settle(&s);
+}
+
 // A wait that ran out is reported until wv_reset, through plans given up and made, and not afterwards.
 void failure()
 {
@@ -230,25 +292,25 @@ void failure()
     make(s);
     const wv::Rec2D rec{};
     CHECK(!res2d_failed(&s));
-    CHECK(res2d_run(&s, 0, 100) == 0 && !res2d_failed(&s));
+    CHECK(run(s, 0, 100) == 0 && !res2d_failed(&s));
     give_up = true;
-    CHECK(res2d_run(&s, 100, 100) == 0 && res2d_failed(&s));
+    CHECK(run(s, 100, 100) == 0 && res2d_failed(&s));
     give_up = false;
-    CHECK(res2d_run(&s, 0, 100, &rec) == 0);  // another plan, another set of buffers
+    CHECK(run(s, 0, 100, &rec) == 0);  // another plan, another set of buffers
     CHECK(res2d_failed(&s));
-    CHECK(res2d_run(&s, 0, 100) == 0);
+    CHECK(run(s, 0, 100) == 0);
     CHECK(res2d_failed(&s));
     last.ctl[2] = 1;
     CHECK(res2d_reset(&s) == 0);
-    CHECK(!res2d_failed(&s) && last.ctl[2] == 0);
-    CHECK(res2d_run(&s, 0, 100) == 0 && !res2d_failed(&s));
-    // a launch from before the reset may still be at it
-    const unsigned before = last.launch;
-    CHECK(res2d_reset(&s) == 0);
-    last.host[1] = before;
     CHECK(!res2d_failed(&s));
+    CHECK(run(s, 0, 100) == 0 && !res2d_failed(&s) && last.ctl[2] == 0);
+    // a launch from before the reset may still be at it
     give_up = true;
-    CHECK(res2d_run(&s, 0, 100) == 0 && res2d_failed(&s));
+    CHECK(res2d_run(&s, 0, 100) == 0);
+    CHECK(res2d_reset(&s) == 0);
+    (void)hipStreamSynchronize(nullptr);
+    CHECK(last.host[1] == last.launch && !res2d_failed(&s));
+    CHECK(run(s, 0, 100) == 0 && res2d_failed(&s));
 }
 
 // A refused check-in leaves the steps to the ordinary kernels until wv_reset, three in a row for good.
@@ -259,28 +321,84 @@ void refusal()
     const wv::Rec2D rec{};
     refuse = true;
     for (int k = 1; k <= 3; k++) {
-        CHECK(res2d_run(&s, 0, 100) == 1 && launches == k);
-        CHECK(res2d_run(&s, 100, 100) == 1 && res2d_run(&s, 200, 100, &rec) == 1 && launches == k);
+        CHECK(run(s, 0, 100) == 1 && launches == k);
+        CHECK(run(s, 100, 100) == 1 && run(s, 200, 100, &rec) == 1 && launches == k);
         CHECK(res2d_reset(&s) == 0);
     }
-    CHECK(res2d_run(&s, 0, 100) == 1 && launches == 3);
+    CHECK(run(s, 0, 100) == 1 && launches == 3);
     wv_solver t;
     make(t);
     launches = 0;
     for (int k = 1; k <= 4; k++) {  // not in a row
         refuse = true;
-        CHECK(res2d_run(&t, 0, 100) == 1);
+        CHECK(run(t, 0, 100) == 1);
         CHECK(res2d_reset(&t) == 0);
+        (void)hipStreamSynchronize(nullptr);
         refuse = false;
-        CHECK(res2d_run(&t, 0, 100) == 0 && launches == 2 * k);
+        CHECK(run(t, 0, 100) == 0 && launches == 2 * k);
     }
     // the same for want of memory
     wv_solver u;
     make(u);
     fail_at = allocations + 2;
-    CHECK(res2d_run(&u, 0, 100) == 1 && res2d_run(&u, 0, 100) == 1);
+    CHECK(run(u, 0, 100) == 1 && run(u, 0, 100) == 1);
     CHECK(res2d_reset(&u) == 0);
-    CHECK(res2d_run(&u, 0, 100) == 0);
+    CHECK(run(u, 0, 100) == 0);
+}
+
+// Launches are queued without waiting for any of them, on two handles in turn; the steps of a refused one
+// and of all behind it are run with the ordinary kernels, in order and once, when the handle is settled.
+void queue()
+{
+    wv_solver a, b;
+    make(a);
+    make(b);
+    CHECK(run(a, 0, 1) == 0 && run(b, 0, 1) == 0);
+    take_notes();
+    for (int k = 0; k < 5; k++) CHECK(res2d_run(&a, 10 * k, 10) == 0 && res2d_run(&b, 7 * k, 7) == 0);
+    CHECK(stream.size() == 10 && ran.empty());
+    CHECK(res2d_queued(&a));
+    work(9);
+    CHECK(!res2d_queued(&a) && res2d_queued(&b));
+    CHECK(res2d_settle(&a) == 0 && stream.size() == 1);  // nothing to wait for
+    CHECK(res2d_settle(&b) == 0 && stream.empty());
+    CHECK(take_notes() == "R0+10 R0+7 R10+10 R7+7 R20+10 R14+7 R30+10 R21+7 R40+10 R28+7 ");
+
+    // the third of five is refused
+    for (int k = 0; k < 5; k++) CHECK(res2d_run(&a, 10 * k, 10) == 0);
+    work(2);
+    refuse = true;
+    work(1);
+    refuse = false;
+    CHECK(res2d_settle(&a) == 1);
+    (void)hipStreamSynchronize(nullptr);
+    CHECK(take_notes() == "R0+10 R10+10 C20 O20+10 C30 O30+10 C40 O40+10 ");
+    CHECK(res2d_settle(&a) == 0 && res2d_run(&a, 50, 10) == 1);
+
+    // wv_reset drops what is queued, refused or not
+    CHECK(res2d_reset(&a) == 0);
+    refuse = true;
+    CHECK(res2d_run(&a, 0, 10) == 0 && res2d_run(&a, 10, 10) == 0);
+    CHECK(res2d_reset(&a) == 0);
+    work(3);
+    refuse = false;
+    CHECK(res2d_run(&a, 0, 10) == 0 && res2d_run(&a, 10, 10) == 0);
+    CHECK(res2d_settle(&a) == 0 && take_notes() == "R0+10 R10+10 ");
+    refuse = true;
+    CHECK(res2d_run(&a, 0, 10) == 0 && res2d_went(&a) == 1 && stream.empty());
+    CHECK(res2d_settle(&a) == 0 && take_notes().empty());
+    refuse = false;
+
+    // another plan while launches of the old one are queued
+    const wv::Rec2D rec{};
+    CHECK(res2d_reset(&a) == 0);
+    CHECK(res2d_run(&a, 0, 10) == 0 && res2d_run(&a, 10, 10, &rec) == 0);
+    CHECK(res2d_settle(&a) == 0 && take_notes() == "R0+10 R10+10 ");
+    CHECK(res2d_run(&a, 20, 10, &rec) == 0);
+    refuse = true;
+    CHECK(res2d_run(&a, 30, 10) == 1 && res2d_settle(&a) == 1);
+    (void)hipStreamSynchronize(nullptr);
+    CHECK(take_notes() == "C20 O20+10 ");
 }
 
 // Read-backs take what device memory there is, down to one item, then pinned host memory.
@@ -335,6 +453,8 @@ int main(int argc, char **argv)
         failure();
     else if (t == "refusal")
         refusal();
+    else if (t == "queue")
+        queue();
     else if (t == "staging")
         staging();
     else

@@ -6,8 +6,10 @@ the other tests hold against the oracle.  Both do the same operations in the sam
 seismograms and final wavefields are equal to the bit: at tile edges (columns 63 .. 129), few and
 many rows, every order, CPML / ABS / rigid edges with and without a free surface, more sources than
 a wavefront and more receivers than a block holds, several rounds of shots, runs cut into pieces,
-and the adjoint's record.
+queued runs, and the adjoint's record.
 """
+import time
+
 import numpy as np
 import pytest
 
@@ -89,6 +91,34 @@ def test_resident_many_sources_and_receivers():
 def test_resident_rounds_of_shots():
     """More shots than the chip holds at once: the blocks take them in rounds."""
     _equal(_case("elastic", 300, 200, 200, 8, 23, 2), 200)
+
+
+def test_resident_runs_are_queued():
+    """wv_run does not wait for the device: four run calls on each of two handles return while the first is at work
+    (0.01 s of a run of about 0.1 s), and both end with the seismograms of handles run one by one."""
+    c = _case("elastic", 300, 200, 6000, 8, 2, 2)
+    ref = cases.make_solver(c)
+    ref.run(0, 6000)
+    want = [ref.seismograms(k) for k in range(2)]
+    hs = [cases.make_solver(c) for _ in range(2)]
+    for h in hs:
+        h.run(0, 6000)
+        h.synchronize()
+        h.reset()
+    t0 = time.perf_counter()
+    for n in range(4):
+        for h in hs:
+            h.run(1500 * n, 1500 * n + (1500 if n < 3 else 1495))
+    for h in hs:
+        h.run(5995, 6000)
+    queued = time.perf_counter() - t0
+    for h in hs:
+        h.synchronize()
+    total = time.perf_counter() - t0
+    assert queued < total / 4, (queued, total)
+    for h in hs:
+        for k in range(2):
+            assert np.array_equal(h.seismograms(k), want[k])
 
 
 def test_resident_record_gives_the_same_gradient():

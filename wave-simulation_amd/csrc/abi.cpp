@@ -51,6 +51,7 @@ wv_solver::~wv_solver()
 int wv_solver::sync_acquisition()
 {
     if (!acq_dirty) return 0;
+    if (const int rc = res2d_settle(this); rc < 0) return rc;
     drop_graph();
     HIP_TRY(hipStreamSynchronize(st));
     free_list(acq_allocs);
@@ -581,6 +582,7 @@ int wv_set_model(wv_solver *s, const float *m0, const float *m1, const float *m2
         s->model_ok = true;
         return WV_OK;
     }
+    if (const int rc = res2d_settle(s); rc < 0) return rc;
     if (s->visco && s->vL == 0) return fail(WV_ESTATE, "the viscoelastic model needs wv_set_relaxation first");
     const wv::Layout2D &L = s->L;
     const int NX = L.NX, NY = L.NY;
@@ -1051,6 +1053,7 @@ int wv_run(wv_solver *s, int t_start, int t_end)
     if (res2d_failed(s)) return fail(WV_EDEVICE, kResidentFailed);
     int rc = s->sync_acquisition();
     if (rc) return rc;
+    if (s->ktiming && (rc = res2d_settle(s)) < 0) return rc;
     HIP_TRY(hipEventRecord(s->ev0, s->st));
     int t = t_start;
     auto eager = [&](int n) -> int {
@@ -1067,8 +1070,9 @@ int wv_run(wv_solver *s, int t_start, int t_end)
         int n = t_end - t;
         if (ck) n = std::min(n, ck - t % ck);
         const wv::Rec2D *rec = adjoint_record(s);
-        if (n >= kResidentSteps && s->use_res && res2d_eligible(s) && (s->variant == V_STRIP || s->physics != wv::ELASTIC) &&
-            (s->use_res > 0 || res2d_expected(s, rec != nullptr))) {
+        // (behind queued launches shorter segments too: the others would wait here for the verdict)
+        if (s->use_res && res2d_eligible(s) && (s->variant == V_STRIP || s->physics != wv::ELASTIC) &&
+            (n >= kResidentSteps || res2d_queued(s)) && (s->use_res > 0 || res2d_expected(s, rec != nullptr))) {
             const int r2 = res2d_run(s, t, n, rec);
             if (r2 < 0) return r2;
             if (r2 == 0) {
@@ -1076,6 +1080,9 @@ int wv_run(wv_solver *s, int t_start, int t_end)
                 continue;
             }
         }
+        if ((rc = res2d_settle(s)) < 0) return rc;
+        // the state was not there yet when the checkpoint was made
+        if (rc == 1 && (rc = adjoint_checkpoint_again(s, t))) return rc;
         // (the persistent kernel is one cooperative launch per segment already: no graph)
         if (K > 0 && n >= K + s->cur && s->variant != V_PERSIST) {
             if (s->cur) {  // graphs start in buffer 0
@@ -1117,6 +1124,7 @@ int wv_run(wv_solver *s, int t_start, int t_end)
 int wv_synchronize(wv_solver *s)
 {
     if (!s || !s->inited) return fail(WV_ESTATE, "not initialised");
+    if (const int rc = res2d_settle(s); rc < 0) return rc;
     HIP_TRY(hipStreamSynchronize(s->st));
     if (res2d_failed(s)) return fail(WV_EDEVICE, kResidentFailed);
     return WV_OK;
@@ -1125,6 +1133,7 @@ int wv_synchronize(wv_solver *s)
 int wv_last_run_ms(wv_solver *s, double *ms)
 {
     if (!s || !s->inited || !s->ran || !ms) return fail(WV_ESTATE, "no run recorded");
+    if (const int rc = res2d_settle(s); rc < 0) return rc;
     HIP_TRY(hipEventSynchronize(s->ev1));
     float f = 0;
     HIP_TRY(hipEventElapsedTime(&f, s->ev0, s->ev1));
@@ -1151,6 +1160,7 @@ int wv_get_seismograms(wv_solver *s, int shot, float *out)
         std::fill(out, out + (size_t)nrec * NT, 0.f);
         return WV_OK;
     }
+    if (const int rc = res2d_settle(s); rc < 0) return rc;
     HIP_TRY(hipStreamSynchronize(s->st));
     if (res2d_failed(s)) return fail(WV_EDEVICE, kResidentFailed);
     HIP_TRY(wv::read_traces(s->stage, s->d_seis, s->rec_total, s->rec_ptr_h[shot], nrec, NT, out, s->st));
@@ -1171,6 +1181,7 @@ static int field_io(wv_solver *s, int shot, int field, float *out, const float *
     }
     if (field < 0 || field >= s->nfields) return fail(WV_EINVAL, "bad field index");
     const wv::Layout2D &L = s->L;
+    if (const int rc = res2d_settle(s); rc < 0) return rc;
     float *d = s->field[s->cur][field] + (size_t)shot * L.plane;
     HIP_TRY(hipStreamSynchronize(s->st));
     if (res2d_failed(s)) return fail(WV_EDEVICE, kResidentFailed);
@@ -1281,11 +1292,13 @@ int wv_tune(wv_solver *s, int nsteps, int *choice)
         if ((rc = s->sync_acquisition())) return rc;
         if (s->variant == V_STRIP || s->physics != wv::ELASTIC) {
             if ((rc = res2d_run(s, 0, 2)) < 0) return rc;
+            if (rc == 0 && (rc = res2d_went(s)) < 0) return rc;
             if (rc == 0) {
                 HIP_TRY(hipEventRecord(s->ev0, s->st));
                 if ((rc = res2d_run(s, 0, nsteps)) < 0) return rc;
                 HIP_TRY(hipEventRecord(s->ev1, s->st));
                 HIP_TRY(hipEventSynchronize(s->ev1));
+                if (rc == 0 && (rc = res2d_went(s)) < 0) return rc;
                 float ms = 0;
                 HIP_TRY(hipEventElapsedTime(&ms, s->ev0, s->ev1));
                 s->use_res = rc == 0 && ms < best ? 1 : 0;

@@ -137,6 +137,34 @@ struct KernelTimer {
     }
 };
 
+// the current state into checkpoint k
+int store_checkpoint(wv_solver *s, int k)
+{
+    AdjointState *a = s->adj;
+    for (int f = 0; f < 5; f++) {
+        if (a->fp16) {
+            unsigned short *h = (unsigned short *)a->ck_fields[k] + (size_t)f * a->fld_n;
+            wv::launch_ckpt_pack(s->field[0][f], h, a->ck_max[k] + (size_t)f * s->cfg.nshots, s->L.plane,
+                                 s->cfg.nshots, s->st);
+        } else {
+            float *d = (float *)a->ck_fields[k] + (size_t)f * a->fld_n;
+            HIP_TRY(hipMemcpyAsync(d, s->field[0][f], a->fld_n * sizeof(float), hipMemcpyDeviceToDevice, s->st));
+        }
+    }
+    if (psi_total(s)) {
+        float *p[8];
+        size_t n[8];
+        psi_list(s, p, n);
+        float *d = a->ck_psi[k];
+        for (int q = 0; q < 8; q++) {
+            HIP_TRY(hipMemcpyAsync(d, p[q], n[q] * sizeof(float), hipMemcpyDeviceToDevice, s->st));
+            d += n[q];
+        }
+    }
+    HIP_TRY(hipGetLastError());
+    return 0;
+}
+
 }  // namespace
 
 void adjoint_destroy(AdjointState *a)
@@ -177,29 +205,16 @@ int adjoint_checkpoint(wv_solver *s, int t)
     }
     const int k = t / a->every;
     if (k >= a->nck) return 0;
-    for (int f = 0; f < 5; f++) {
-        if (a->fp16) {
-            unsigned short *h = (unsigned short *)a->ck_fields[k] + (size_t)f * a->fld_n;
-            wv::launch_ckpt_pack(s->field[0][f], h, a->ck_max[k] + (size_t)f * s->cfg.nshots, s->L.plane,
-                                 s->cfg.nshots, s->st);
-        } else {
-            float *d = (float *)a->ck_fields[k] + (size_t)f * a->fld_n;
-            HIP_TRY(hipMemcpyAsync(d, s->field[0][f], a->fld_n * sizeof(float), hipMemcpyDeviceToDevice, s->st));
-        }
-    }
-    if (psi_total(s)) {
-        float *p[8];
-        size_t n[8];
-        psi_list(s, p, n);
-        float *d = a->ck_psi[k];
-        for (int q = 0; q < 8; q++) {
-            HIP_TRY(hipMemcpyAsync(d, p[q], n[q] * sizeof(float), hipMemcpyDeviceToDevice, s->st));
-            d += n[q];
-        }
-    }
-    HIP_TRY(hipGetLastError());
-    a->have[k] = 1;
-    return 0;
+    const int rc = store_checkpoint(s, k);
+    if (rc == 0) a->have[k] = 1;
+    return rc;
+}
+
+int adjoint_checkpoint_again(wv_solver *s, int t)
+{
+    const AdjointState *a = s->adj;
+    if (!a || !a->every || a->store || t % a->every || t / a->every >= a->nck || !a->have[t / a->every]) return 0;
+    return store_checkpoint(s, t / a->every);
 }
 
 void adjoint_run_begin(wv_solver *s, int t_start)
@@ -239,6 +254,7 @@ int wv_set_checkpointing(wv_solver *s, int every, int fp16)
     if (!wv::strip2d_fits(s->L)) return fail(WV_EINVAL, "grid too large for the adjoint kernels (field plane of 2 GiB or more)");
     if (!s->adj) s->adj = new AdjointState();
     AdjointState *a = s->adj;
+    if (const int rc = res2d_settle(s); rc < 0) return rc;
     HIP_TRY(hipStreamSynchronize(s->st));
     if (every && every == a->every && (fp16 != 0) == a->fp16 && s->variant != V_SINGLE) {
         // same layout: keep the checkpoint buffers
@@ -338,6 +354,7 @@ int wv_set_adjoint_store(wv_solver *s, double max_gib)
 {
     if (!s || !s->inited) return fail(WV_ESTATE, "wv_set_adjoint_store before wv_init");
     if (!(max_gib == max_gib)) return fail(WV_EINVAL, "bad budget");
+    if (const int rc = res2d_settle(s); rc < 0) return rc;
     if (!s->adj) s->adj = new AdjointState();
     s->adj->store_gib = max_gib;
     s->adj->every = 0;  // the next wv_set_checkpointing chooses the memory plan again
@@ -372,13 +389,15 @@ int wv_run_adjoint(wv_solver *s)
     }
     if (!s || !s->inited || !s->adj || !s->adj->every) return fail(WV_ESTATE, "checkpointing is not enabled");
     AdjointState *a = s->adj;
-    if (res2d_failed(s)) return fail(WV_EDEVICE, kResidentFailed);
     if (!a->forward_done) return fail(WV_ESTATE, "wv_run_adjoint needs a checkpointed forward run over [0, NT)");
     for (int k = 0; k < a->nck; k++)
         if (!a->have[k]) return fail(WV_ESTATE, "missing checkpoint");
     if (a->store && (s->variant != V_STRIP || s->tile_y / 4 != a->rec.srows))
         return fail(WV_ESTATE, "the kernel variant changed after wv_set_checkpointing: repeat it and the forward run");
     int rc;
+    if ((rc = res2d_settle(s)) < 0) return rc;
+    HIP_TRY(hipStreamSynchronize(s->st));
+    if (res2d_failed(s)) return fail(WV_EDEVICE, kResidentFailed);
     if ((rc = s->sync_acquisition())) return rc;
     const wv::Layout2D &L = s->L;
     const int NT = s->cfg.NT, K = a->every, ns = s->cfg.nshots, H = s->H;

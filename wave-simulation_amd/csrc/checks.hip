@@ -192,6 +192,7 @@ int wv_check_parameters(const char *dimension, const char *type, const wv_config
 int wv_check_finite(wv_solver *s)
 {
     if (!s || !s->inited) return fail(WV_ESTATE, "not initialised");
+    if (const int rc = res2d_settle(s); rc < 0) return rc;
     wv::StateBuffers bufs;
     state_buffers(s, bufs);
     if (!s->d_flag) {
@@ -217,6 +218,7 @@ int wv_check_finite_noalloc(wv_solver *s, long long *nonfinite)
 {
     if (nonfinite) *nonfinite = 0;
     if (!s || !s->inited) return fail(WV_ESTATE, "not initialised");
+    if (const int rc = res2d_settle(s); rc < 0) return rc;
     wv::StateBuffers bufs;
     state_buffers(s, bufs);
     if (bufs.overflow)

@@ -303,6 +303,8 @@ const wv::Rec2D *adjoint_record(const wv_solver *s);
 // called by wv_run: at its start, before step t (t a multiple of the interval), at its end
 void adjoint_run_begin(wv_solver *s, int t_start);
 int adjoint_checkpoint(wv_solver *s, int t);
+// the checkpoint made before step t, if one was, from the state there is now
+int adjoint_checkpoint_again(wv_solver *s, int t);
 void adjoint_run_done(wv_solver *s, int t_end);
 
 // resident2d.cpp: the resident 2D time loop
@@ -311,6 +313,12 @@ void res2d_acquisition_changed(wv_solver *s);
 bool res2d_eligible(const wv_solver *s);
 int res2d_run(wv_solver *s, int t0, int nsteps, const wv::Rec2D *rec = nullptr, float *snap = nullptr,
               long long snap_field = 0, long long snap_step = 0);
+// Launches are enqueued without a look at whether they will go. Whatever reads or changes the state, what the
+// ordinary kernels work with, or the clock of a run settles them first: waits where a verdict is not in and
+// has the ordinary kernels run the steps of refused launches. 1: it did; 0: there were none; < 0: error.
+int res2d_settle(wv_solver *s);
+int res2d_went(wv_solver *s);     // the same without running the steps of refused launches
+bool res2d_queued(wv_solver *s);  // a verdict is not in, nor comes at once
 size_t res2d_bytes(wv_solver *s, int srow);  // device bytes its buffers will want
 bool res2d_expected(wv_solver *s, bool rec);
 bool res2d_failed(const wv_solver *s);

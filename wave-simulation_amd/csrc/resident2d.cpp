@@ -1,8 +1,8 @@
 // Host side of the resident 2D time loop: launch plan, acquisition lists, exchange buffer, the
 // hand-shake with a launch.
-#include <sched.h>
-
 #include <algorithm>
+#include <chrono>
+#include <mutex>
 
 #include "handle.hpp"
 #include "resident2d.hpp"
@@ -151,6 +151,12 @@ hipError_t launch_res2d(int physics, int order, const Res2DPlan &plan, const Lay
 
 }  // namespace wv
 
+// A launch and the steps it stands for.
+struct Res2DQueued {
+    int t0, nsteps;
+    unsigned launch;
+};
+
 struct Res2DState {
     wv::Res2DPlan plan;
     double gain = 0.0;  // estimated step time of the two-launch kernels over that of the plan
@@ -162,13 +168,15 @@ struct Res2DState {
     unsigned long long *xch = nullptr;
     unsigned *ctl = nullptr;
     float *psi = nullptr;
-    unsigned *host = nullptr;  // pinned, one for the handle's life: see Res2DArgs
+    unsigned long long *host = nullptr;  // pinned, one for the handle's life: see Res2DArgs
     int words = 0, phase1 = 0;  // exchange words of a block
     unsigned tag = 1, arrived = 0;
     unsigned launches = 0;  // made in the handle's life
     unsigned first = 1;     // the first one since the last wv_reset
     bool off = false;       // the ordinary kernels run the steps until the next wv_reset
     int refused = 0;        // check-ins refused in a row
+    std::vector<Res2DQueued> queued;  // launches not known to have gone, in order
+    std::mutex lock;                  // of `queued`: results may be read from several threads
     hipEvent_t ev[2] = {};  // per-kernel timing
     bool timed = false;     // the timed run calls went through the resident loop
 };
@@ -200,6 +208,94 @@ bool res2d_eligible(const wv_solver *s)
     return s->cfg.tile_y == 0 && (s->cfg.path == WV_PATH_FUSED || (s->cfg.path == WV_PATH_STRIP && s->physics == wv::ELASTIC));
 }
 
+// What is known of the queued launches: 0 some verdict is not in (launches that went are taken off), 1 all
+// went, 2 some were refused.
+static int res_verdicts(Res2DState *r)
+{
+    std::vector<Res2DQueued> &q = r->queued;
+    if (q.empty()) return 1;
+    const unsigned long long w = __atomic_load_n(r->host, __ATOMIC_ACQUIRE);
+    const unsigned first = (unsigned)(w >> 32), v = (unsigned)w;
+    if (v & 1) {
+        // (a refusal from before the latest wv_reset concerns none of these)
+        if ((int)(first - q.front().launch) >= 0 && v == 2 * q.back().launch + 1) return 2;
+        return 0;
+    }
+    size_t n = 0;
+    while (n < q.size() && (int)(v - 2 * q[n].launch) >= 0) n++;
+    if (n) r->refused = 0;
+    q.erase(q.begin(), q.begin() + n);
+    return q.empty() ? 1 : 0;
+}
+
+// Waits for the verdicts. 0: all queued launches went; 1: some were refused, and *redo has them in order
+// (the loop is off then); < 0: error.
+static int res_settle(wv_solver *s, std::vector<Res2DQueued> *redo)
+{
+    Res2DState *r = s->res;
+    int v = res_verdicts(r);
+    if (v == 0) {
+        HIP_TRY(hipStreamSynchronize(s->st));
+        v = res_verdicts(r);
+    }
+    if (v == 1) return 0;
+    std::vector<Res2DQueued> q;
+    q.swap(r->queued);
+    if (v == 0) return fail(WV_EDEVICE, "the resident time loop ended without a verdict");
+    const unsigned first = (unsigned)(__atomic_load_n(r->host, __ATOMIC_ACQUIRE) >> 32);
+    for (const Res2DQueued &e : q)
+        if ((int)(e.launch - first) >= 0) redo->push_back(e);
+    // something else holds the GPU
+    r->off = true;
+    r->refused++;
+    return 1;
+}
+
+// The steps of refused launches, with the ordinary kernels, and the checkpoints between them.
+static int res_redo(wv_solver *s, const std::vector<Res2DQueued> &q)
+{
+    for (const Res2DQueued &e : q) {
+        int rc = adjoint_checkpoint_again(s, e.t0);
+        if (rc) return rc;
+        wv::launch_set(s->d_tbase, e.t0, s->st);
+        if ((rc = s->enqueue_steps(e.nsteps, false))) return rc;
+    }
+    return 0;
+}
+
+int res2d_settle(wv_solver *s)
+{
+    if (!s->res) return 0;
+    std::lock_guard<std::mutex> hold(s->res->lock);
+    std::vector<Res2DQueued> redo;
+    int rc = res_settle(s, &redo);
+    if (rc == 1 && (rc = res_redo(s, redo)) == 0) {
+        HIP_TRY(hipEventRecord(s->ev1, s->st));
+        return 1;
+    }
+    return rc;
+}
+
+int res2d_went(wv_solver *s)
+{
+    if (!s->res) return 0;
+    std::lock_guard<std::mutex> hold(s->res->lock);
+    std::vector<Res2DQueued> refused;
+    return res_settle(s, &refused);
+}
+
+bool res2d_queued(wv_solver *s)
+{
+    if (!s->res) return false;
+    std::lock_guard<std::mutex> hold(s->res->lock);
+    // (a launch on an idle stream begins within tens of microseconds)
+    const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(200);
+    int v;
+    while ((v = res_verdicts(s->res)) == 0 && std::chrono::steady_clock::now() < until) {
+    }
+    return v == 0;
+}
+
 // The plan for the handle (rows per wavefront as the record's strips when it is written); false:
 // the resident loop does not take this problem.
 static bool res_plan(wv_solver *s, int srow)
@@ -208,6 +304,9 @@ static bool res_plan(wv_solver *s, int srow)
     Res2DState *r = s->res;
     if (r->off) return false;
     if (r->planned && r->srow == srow) return (bool)r->plan;
+    // the queued launches use the buffers of the plan that goes (refused ones: the caller finds the loop
+    // off, and settles before it runs anything)
+    if (!r->queued.empty() && (hipStreamSynchronize(s->st) != hipSuccess || res_verdicts(r) != 1)) return false;
     s->free_list(r->acq_allocs);
     s->free_list(r->allocs);
     r->lists = false;
@@ -258,8 +357,8 @@ static bool res_buffers(wv_solver *s)
     unsigned long long *xch = nullptr;
     unsigned *ctl = nullptr;
     float *psi = nullptr;
-    unsigned *host = nullptr;
-    if (s->dalloc(&xch, words * p.blocks(), got) || s->dalloc(&ctl, 3, got) ||
+    unsigned long long *host = nullptr;
+    if (s->dalloc(&xch, words * p.blocks(), got) || s->dalloc(&ctl, 4, got) ||
         (npsi && s->dalloc(&psi, npsi, got)) ||
         (!r->host && hipHostMalloc((void **)&host, 64, hipHostMallocDefault) != hipSuccess)) {
         (void)hipGetLastError();
@@ -321,8 +420,8 @@ static bool res_lists(wv_solver *s)
     return true;
 }
 
-// nsteps steps from t0 in one launch.  0: done (enqueued and started); 1: not started (the caller
-// runs the steps with the ordinary kernels); < 0: error.
+// nsteps steps from t0 in one launch.  0: enqueued (timed: done); 1: not (the caller settles and runs the steps
+// with the ordinary kernels); < 0: error.
 int res2d_run(wv_solver *s, int t0, int nsteps, const wv::Rec2D *rec, float *snap, long long snap_field,
               long long snap_step)
 {
@@ -381,35 +480,21 @@ int res2d_run(wv_solver *s, int t0, int nsteps, const wv::Rec2D *rec, float *sna
     }
     const int rounds = (s->cfg.nshots + p.conc - 1) / p.conc;
     r->tag += (unsigned)(rounds * nsteps);
-    // the launch says whether all its blocks came in before it touched the state
-    volatile unsigned *h = r->host;
-    const unsigned go = 2 * X.launch, stop = go + 1;
-    for (int n = 1; h[0] != go && h[0] != stop; n++) {
-        if ((n & 255) == 0) {
-            const hipError_t q = hipStreamQuery(s->st);
-            if (q != hipSuccess && q != hipErrorNotReady) HIP_TRY(q);
-            if (q == hipSuccess && h[0] != go && h[0] != stop)
-                return fail(WV_EDEVICE, "the resident time loop ended without a verdict");
-        }
-        sched_yield();
+    {
+        std::lock_guard<std::mutex> hold(r->lock);
+        (void)res_verdicts(r);
+        r->queued.push_back({t0, nsteps, X.launch});
     }
-    if (h[0] == go) {
-        r->refused = 0;
-        if (e0) {
-            HIP_TRY(hipEventRecord(e1, s->st));
-            HIP_TRY(hipEventSynchronize(e1));
-            float ms = 0;
-            HIP_TRY(hipEventElapsedTime(&ms, e0, e1));
-            s->kms[0] += ms;
-            s->klaunch[0] += nsteps;  // counted per time step
-            r->timed = true;
-        }
-        return 0;
-    }
-    // something else holds the GPU
-    r->off = true;
-    r->refused++;
-    return 1;
+    if (!e0) return 0;
+    HIP_TRY(hipEventRecord(e1, s->st));
+    HIP_TRY(hipEventSynchronize(e1));
+    if (const int rc = res2d_went(s)) return rc;
+    float ms = 0;
+    HIP_TRY(hipEventElapsedTime(&ms, e0, e1));
+    s->kms[0] += ms;
+    s->klaunch[0] += nsteps;  // counted per time step
+    r->timed = true;
+    return 0;
 }
 
 // Whether the planner expects the resident loop to be the faster one for the handle's run calls.
@@ -421,7 +506,7 @@ bool res2d_expected(wv_solver *s, bool rec) { return res_plan(s, rec ? s->tile_y
 bool res2d_failed(const wv_solver *s)
 {
     if (!s->res || !s->res->host) return false;
-    const unsigned launch = ((volatile unsigned *)s->res->host)[1];
+    const unsigned launch = (unsigned)__atomic_load_n(s->res->host + 1, __ATOMIC_ACQUIRE);
     return launch && (int)(launch - s->res->first) >= 0;
 }
 
@@ -432,9 +517,12 @@ int res2d_reset(wv_solver *s)
 {
     Res2DState *r = s->res;
     if (!r) return 0;
+    std::lock_guard<std::mutex> hold(r->lock);
+    (void)res_verdicts(r);
+    r->queued.clear();
     r->first = r->launches + 1;
     if (r->refused < 3) r->off = false;
-    if (r->xch) HIP_TRY(hipMemsetAsync(r->ctl + 2, 0, sizeof(unsigned), s->st));
+    if (r->xch) HIP_TRY(hipMemsetAsync(r->ctl + 2, 0, 2 * sizeof(unsigned), s->st));
     return 0;
 }
 

@@ -24,9 +24,11 @@ struct Res2DArgs {
     int words, phase1;         // exchange words of a block; first one of the stress-type phase
     unsigned long long *xch;   // [block][words]: value in the low half, tag in the high half
     unsigned tag0;             // tag of the launch's first step
-    unsigned *ctl;             // [0] blocks arrived (all launches), [1] verdict, [2] a wait ran out
+    unsigned *ctl;             // [0] blocks arrived (all launches), [1] verdict, [2] a wait ran out,
+                               // [3] the launch whose refusal those queued behind it share
     unsigned arrive, launch;   // value of ctl[0] when all blocks of this launch are in; launch number
-    volatile unsigned *host;   // pinned: [0] verdict of the launch, [1] the launch whose wait ran out last
+    unsigned long long *host;  // pinned: [0] the latest verdict: 2 launch (+ 1: refused), and in the high half
+                               // the launch whose refusal it shares; [1] the launch whose wait ran out last
     const int *bsrc_ptr, *bsrc, *brec_ptr, *brec;  // acquisition lists per (shot, tile) of this plan
     float *psi;                // memory variables of the resident tiles, [block][wavefront][psi_wave floats]
     float *snap;               // elastic: segment record (Snap2D planes of step t0), or nullptr

@@ -20,8 +20,9 @@
 // (likewise for the stress slots).  The exchange after the last step of a shot is therefore kept.
 //
 // Every wait ends: the launch is cooperative, the blocks meet once before they touch any state and
-// give the launch up together when some block has not come in after START_TICKS, and later waits
-// end with an error after WAIT_TICKS.
+// give the launch up together when some block has not come in after RES_START_TICKS, and later waits
+// end with an error after RES_WAIT_TICKS.  The host asks for the verdict only where it waits for the
+// stream anyway, and has the ordinary kernels run the steps of a refused launch then.
 //
 // Arithmetic: the operations of the row-strip kernels (elastic) and of the tiled ones
 // (acoustic, SH, TM-EM) in their order, so a run may change between them at any step.
@@ -96,21 +97,25 @@ __device__ __forceinline__ unsigned agent_load(const unsigned *p)
 }
 
 // The blocks of a launch meet before they touch any state: the last one in (or the first whose
-// patience runs out) decides for all.  True: go.
+// patience runs out) decides for all.  A launch queued behind a refused one is refused at once, since
+// the state is not the one it was meant for; the host runs the steps of all of them.  True: go.
 __device__ __forceinline__ bool res_check_in(const Res2DArgs &X, int *s_go)
 {
     if (threadIdx.x == 0) {
         const unsigned go = 2 * X.launch, stop = 2 * X.launch + 1;
         const unsigned n = __hip_atomic_fetch_add(X.ctl, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
         const unsigned long long t0 = wall_clock64();
+        const unsigned behind = agent_load(X.ctl + 3);
         unsigned v = agent_load(X.ctl + 1);
-        unsigned want = n == X.arrive ? go : 0;
+        unsigned want = behind ? stop : n == X.arrive ? go : 0;
         while (v != go && v != stop) {
             if (!want && wall_clock64() - t0 > RES_START_TICKS) want = stop;
             if (want) {
                 if (__hip_atomic_compare_exchange_strong(X.ctl + 1, &v, want, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                                          __HIP_MEMORY_SCOPE_AGENT)) {
-                    __hip_atomic_store(const_cast<unsigned *>(X.host), want, __ATOMIC_RELAXED,
+                    const unsigned first = want == go ? 0 : behind ? behind : X.launch;
+                    if (first) __hip_atomic_store(X.ctl + 3, first, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    __hip_atomic_store(X.host, ((unsigned long long)first << 32) | want, __ATOMIC_RELAXED,
                                        __HIP_MEMORY_SCOPE_SYSTEM);
                     v = want;
                 }
@@ -721,7 +726,7 @@ __global__ __launch_bounds__(MAXT, MINW) void res2d(Res2DKernArgs KA)
         if (bad) {
             if (tid == 0) {
                 __hip_atomic_store(KA.X.ctl + 2, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_store(const_cast<unsigned *>(KA.X.host) + 1, KA.X.launch, __ATOMIC_RELAXED,
+                __hip_atomic_store(KA.X.host + 1, (unsigned long long)KA.X.launch, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_SYSTEM);
             }
             return;
