@@ -93,6 +93,36 @@ def test_resident_rounds_of_shots():
     _equal(_case("elastic", 300, 200, 200, 8, 23, 2), 200)
 
 
+@pytest.mark.parametrize("physics", ["elastic", "acoustic", "sh", "tmem"])
+@pytest.mark.parametrize("axis,cell", [("x", (20, 100)), ("y", (75, 20))])
+def test_resident_infinities_beside_the_frame(physics, axis, cell):
+    """A field that overflows: cells that a CPML frame only shares a tile or a wavefront with have no memory
+    variables, so an infinite derivative stays one, as in the two-launch kernels (0 times infinity is NaN)."""
+    NX, NY, NT = 150, 140, 20
+    c = _case(physics, NX, NY, NT, 4, 1, 2)
+    # a field that is differentiated along the axis, and receivers of what its derivative goes to
+    field = {"x": {"elastic": 2, "acoustic": 2, "sh": 1, "tmem": 1},
+             "y": {"elastic": 4, "acoustic": 2, "sh": 2, "tmem": 0}}[axis][physics]
+    sh = c.shots[0]
+    xy = [(x, y) for y in range(cell[1] - 6, cell[1] + 7) for x in range(cell[0] - 6, cell[0] + 7)]
+    sh.rec_index = np.array([x + y * NX for x, y in xy])
+    sh.rec_type = np.full(len(xy), {"sh": 4, "elastic": 2, "tmem": 1, "acoustic": 2 if axis == "x" else 3}[physics],
+                          np.int32)
+    seis, fields = [], []
+    for kw in (dict(), dict(path=TWO[physics], tile_y=16)):
+        s = cases.make_solver(c, **kw)
+        w = s.wavefield(field, 0)
+        w[cell[0] + cell[1] * NX] = np.inf
+        s.set_wavefield(field, w, 0)
+        s.run(0, NT)
+        seis.append(s.seismograms(0))
+        fields.append([s.wavefield(k, 0) for k in range(5 if physics == "elastic" else 3)])
+    assert np.isinf(seis[1]).any()
+    assert np.array_equal(seis[0], seis[1], equal_nan=True)
+    for a, b in zip(*fields):
+        assert np.array_equal(a, b, equal_nan=True)
+
+
 def test_resident_runs_are_queued():
     """wv_run does not wait for the device: four run calls on each of two handles return while the first is at work
     (0.01 s of a run of about 0.1 s), and both end with the seismograms of handles run one by one."""
