@@ -311,8 +311,7 @@ void adjoint_run_done(wv_solver *s, int t_end);
 void res2d_destroy(wv_solver *s);
 void res2d_acquisition_changed(wv_solver *s);
 bool res2d_eligible(const wv_solver *s);
-int res2d_run(wv_solver *s, int t0, int nsteps, const wv::Rec2D *rec = nullptr, float *snap = nullptr,
-              long long snap_field = 0, long long snap_step = 0);
+int res2d_run(wv_solver *s, int t0, int nsteps, const wv::Rec2D *rec = nullptr);
 // Launches are enqueued without a look at whether they will go. Whatever reads or changes the state, what the
 // ordinary kernels work with, or the clock of a run settles them first: waits where a verdict is not in and
 // has the ordinary kernels run the steps of refused launches. 1: it did; 0: there were none; < 0: error.

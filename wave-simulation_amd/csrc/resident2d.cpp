@@ -146,7 +146,7 @@ hipError_t launch_res2d(int physics, int order, const Res2DPlan &plan, const Lay
     g.rec = rec ? *rec : Rec2D{};
     g.st = stream;
     g.lds = res_lds(physics, order / 2, plan.srow * plan.wmax);
-    return res_dispatch(physics, order, rec != nullptr || X.snap != nullptr, g);
+    return res_dispatch(physics, order, rec != nullptr, g);
 }
 
 }  // namespace wv
@@ -422,10 +422,9 @@ static bool res_lists(wv_solver *s)
 
 // nsteps steps from t0 in one launch.  0: enqueued (timed: done); 1: not (the caller settles and runs the steps
 // with the ordinary kernels); < 0: error.
-int res2d_run(wv_solver *s, int t0, int nsteps, const wv::Rec2D *rec, float *snap, long long snap_field,
-              long long snap_step)
+int res2d_run(wv_solver *s, int t0, int nsteps, const wv::Rec2D *rec)
 {
-    if (!res_plan(s, rec || snap ? s->tile_y / 4 : 0)) return 1;
+    if (!res_plan(s, rec ? s->tile_y / 4 : 0)) return 1;
     Res2DState *r = s->res;
     const wv::Res2DPlan &p = r->plan;
     if (!res_buffers(s) || !res_lists(s)) {
@@ -458,9 +457,6 @@ int res2d_run(wv_solver *s, int t0, int nsteps, const wv::Rec2D *rec, float *sna
     X.brec_ptr = r->brec_ptr;
     X.brec = r->brec;
     X.psi = r->psi;
-    X.snap = snap;
-    X.snap_field = snap_field;
-    X.snap_step = snap_step;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (s->ktiming) {
         for (auto &ev : r->ev)

@@ -31,8 +31,6 @@ struct Res2DArgs {
                                // the launch whose refusal it shares; [1] the launch whose wait ran out last
     const int *bsrc_ptr, *bsrc, *brec_ptr, *brec;  // acquisition lists per (shot, tile) of this plan
     float *psi;                // memory variables of the resident tiles, [block][wavefront][psi_wave floats]
-    float *snap;               // elastic: segment record (Snap2D planes of step t0), or nullptr
-    long long snap_field, snap_step;  // floats between two recorded sums / two steps
 };
 
 // Everything a launch is handed, one kernel argument: the time loop reads it from the argument

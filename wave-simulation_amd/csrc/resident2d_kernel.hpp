@@ -646,20 +646,11 @@ __global__ __launch_bounds__(MAXT, MINW) void res2d(Res2DKernArgs KA)
         };
         using c0 = std::integral_constant<int, 0>;
         using c1 = std::integral_constant<int, 1>;
-        // recorded sums of a phase: the run's record, or the segment's planes
-        auto keep = [&](auto first, int st, int tt, const auto &rh) {
+        // the adjoint's record of a phase's sums
+        auto keep = [&](auto first, int tt, const auto &rh) {
             constexpr int F0 = decltype(first)::value, N = F0 ? 3 : 2;
-            const res_args G = fresh_args(G0);
             const int lane = fresh_lane(tid & 63), ya = y0 + fresh_uniform(wave_) * S;
-            if (G->R.h) record_strips<S, N>(KA.R, KA.L, KA.X.nshots, tt, F0, shot, x0, ya, lane, rh);
-            if (G->X.snap)
-#pragma unroll
-                for (int f = 0; f < N; f++)
-#pragma unroll
-                    for (int r = 0; r < S; r++)
-                        if (ya + r < NY && xin)
-                            (KA.X.snap + st * KA.X.snap_step + (F0 + f) * KA.X.snap_field + so + KA.L.at(x0, ya + r))[lane] =
-                                rh[f][r];
+            record_strips<S, N>(KA.R, KA.L, KA.X.nshots, tt, F0, shot, x0, ya, lane, rh);
         };
 
         load_psi(0);
@@ -676,7 +667,7 @@ __global__ __launch_bounds__(MAXT, MINW) void res2d(Res2DKernArgs KA)
                 send(c0{});
                 store_psi(0);
                 load_psi(1);
-                if constexpr (REC) keep(c0{}, st, tt, rh);
+                if constexpr (REC) keep(c0{}, tt, rh);
             }
             recv(c0{});
             block_sync_lds();
@@ -732,7 +723,7 @@ __global__ __launch_bounds__(MAXT, MINW) void res2d(Res2DKernArgs KA)
                     const int id = receiver(G, e, o1, o2);
                     record_sample(G, id, tt, o1, o2);
                 }
-                if constexpr (REC) keep(std::integral_constant<int, 2>{}, st, tt, rh);
+                if constexpr (REC) keep(std::integral_constant<int, 2>{}, tt, rh);
             }
             recv(c1{});
             block_sync_lds();
