@@ -173,6 +173,14 @@ int wv_set_wavefield(wv_solver *s, int shot, int field, const float *in);
  * No counterpart in the reference. */
 int wv_tune(wv_solver *s, int nsteps, int *choice);
 
+/* The resident loop's division of the work, for tests and measurements (runs give the same bits with
+ * every one): takes rows per wavefront (1, 2, 4 or 8) and wavefronts per block (1..16) for the handle's
+ * following runs, 0 = the planner's choice, and reports {rows per wavefront, wavefronts per block, shots
+ * in flight} in plan[3] (may be NULL).  Runs with the adjoint's per-step record take their rows from the
+ * record.  WV_EINVAL where the loop does not take the handle's runs or no such plan fits the device.
+ * No counterpart in the reference. */
+int wv_resident_plan(wv_solver *s, int rows, int waves, int *plan);
+
 /* elapsed GPU time [ms] of the last wv_run (hipEvents on the handle's stream) */
 int wv_last_run_ms(wv_solver *s, double *ms);
 

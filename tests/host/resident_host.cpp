@@ -401,6 +401,27 @@ void queue()
     CHECK(take_notes() == "C20 O20+10 ");
 }
 
+// A division of the work asked for is taken, or refused without a trace.
+void plan()
+{
+    wv_solver s;
+    make(s);
+    int p[3];
+    CHECK(wv_resident_plan(&s, 0, 0, p) == WV_OK);
+    const int free_choice[3] = {p[0], p[1], p[2]};
+    for (int rows : {1, 2, 4, 8}) {
+        CHECK(wv_resident_plan(&s, rows, 8, p) == WV_OK && p[0] == rows && p[1] == 8 && p[2] == 2);
+        CHECK(res2d_expected(&s, false) && run(s, 0, 10) == 0 && last.nwv == 8);
+    }
+    CHECK(wv_resident_plan(&s, 8, 16, p) == WV_EINVAL);  // 8 rows: 8 wavefronts at most
+    CHECK(wv_resident_plan(&s, 1, 3, p) == WV_EINVAL);   // lower than a halo
+    CHECK(wv_resident_plan(&s, 3, 0, p) == WV_EINVAL && wv_resident_plan(&s, 4, 17, p) == WV_EINVAL);
+    CHECK(run(s, 0, 10) == 0 && last.nwv == 8);
+    CHECK(wv_resident_plan(&s, 0, 0, nullptr) == WV_OK && run(s, 0, 10) == 0 && last.nwv == free_choice[1]);
+    s.cfg.tile_y = 16;
+    CHECK(wv_resident_plan(&s, 0, 0, p) == WV_EINVAL);
+}
+
 // Read-backs take what device memory there is, down to one item, then pinned host memory.
 void staging()
 {
@@ -455,6 +476,8 @@ int main(int argc, char **argv)
         refusal();
     else if (t == "queue")
         queue();
+    else if (t == "plan")
+        plan();
     else if (t == "staging")
         staging();
     else

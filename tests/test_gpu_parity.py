@@ -120,10 +120,17 @@ def test_batched_equals_single_shot():
         assert np.array_equal(batched[k], single)
 
 
-def test_graph_segments_equal_eager():
-    c = cases.elastic_c2(N=96, NT=230, W=12)
-    eager = _gpu_all(c)[0]
-    graph = _gpu_all(c, steps_per_graph=50)[0]
+@pytest.mark.parametrize("case,path", [("elastic", "fused"), ("elastic", "phased"), ("elastic", "strip"),
+                                       ("acoustic", "phased"), ("tmem", "phased"), ("tmem", "strip"),
+                                       ("sh", "phased")])
+def test_graph_segments_equal_eager(case, path):
+    """(An explicit tile height: handles without one may run in the resident loop, which launches no graphs.)"""
+    c = {"elastic": lambda: cases.elastic_c2(N=96, NT=230, W=12), "acoustic": lambda: cases.acoustic_c1(N=100, NT=230),
+         "tmem": lambda: cases.tmem_c3(NX=150, NY=90, NT=230, nshots=2, block=10, W=10),
+         "sh": lambda: cases.sh_2d(NT=230, nshots=2)}[case]()
+    eager = _gpu_all(c, path=path, tile_y=16)[0]
+    graph = _gpu_all(c, path=path, tile_y=16, steps_per_graph=50)[0]
+    assert np.abs(eager).max() > 0
     assert np.array_equal(eager, graph)
 
 

@@ -25,7 +25,7 @@ def _case(physics, NX, NY, NT, order, nshots, damping, fs=0, W=8, ops=None):
         c = cases.visco_2d(NX=NX, NY=NY, NT=NT, nshots=nshots, order=order, W=W, damping=damping, free_surface=fs)
         c.type, c.visco = "elastic", None
     elif physics == "sh":
-        c = cases.sh_2d(NX=NX, NY=NY, NT=NT, nshots=nshots, order=order, W=W, damping=damping)
+        c = cases.sh_2d(NX=NX, NY=NY, NT=NT, nshots=nshots, order=order, W=W, damping=damping, free_surface=fs)
     elif physics == "tmem":
         c = cases.viscotmem_2d(NX=NX, NY=NY, NT=NT, nshots=nshots, order=order, W=W, damping=damping)
         c.type, c.visco = "tmem", None
@@ -35,8 +35,10 @@ def _case(physics, NX, NY, NT, order, nshots, damping, fs=0, W=8, ops=None):
     return c
 
 
-def _equal(c, NT, pieces=None, **kw):
+def _equal(c, NT, pieces=None, plan=None, **kw):
     a = cases.make_solver(c, **kw)
+    if plan:
+        assert a.resident_plan(*plan)[:2] == plan
     b = cases.make_solver(c, path=TWO[c.type], tile_y=16)
     cuts = [0] + (pieces or []) + [NT]
     for t0, t1 in zip(cuts[:-1], cuts[1:]):
@@ -55,6 +57,23 @@ def _equal(c, NT, pieces=None, **kw):
                                                  (8, 190, 41, 1), (10, 128, 61, 2), (12, 131, 130, 2)])
 def test_resident_equals_two_launch(physics, order, NX, NY, damping):
     _equal(_case(physics, NX, NY, 90, order, 2, damping), 90)
+
+
+@pytest.mark.parametrize("physics", ["elastic", "acoustic", "sh", "tmem"])
+@pytest.mark.parametrize("rows", [1, 2, 4, 8])
+@pytest.mark.parametrize("order,tile,damping,fs", [(2, "least", 2, 0), (8, "least", 1, 0), (8, "odd", 2, 0),
+                                                   (8, "most", 2, 1), (12, "most", 2, 0), (4, "odd", 1, 1),
+                                                   (12, "odd", 0, 0)])
+def test_resident_rows_per_wavefront(physics, rows, order, tile, damping, fs):
+    """Every kernel variant, with the smallest block (one halo high), one of an odd number of wavefronts and the
+    largest, over tiles that are cut at the right and at the bottom, inside a wavefront's rows too."""
+    waves = {"least": max(1, -(-order // 2 // rows)), "odd": 5 if rows < 4 else 3, "most": 16 if rows < 8 else 8}[tile]
+    if waves * rows < order // 2:
+        waves = 7
+    R = waves * rows
+    NY = max(3 * order, 2 * R + R // 2 + 3, 45)
+    c = _case(physics, 150, NY, 150, order, 2, damping, fs=fs if physics != "tmem" else 0, W=10)
+    _equal(c, 150, pieces=[25], plan=(rows, waves))
 
 
 @pytest.mark.parametrize("physics", ["elastic", "acoustic"])
@@ -94,12 +113,13 @@ def test_resident_rounds_of_shots():
 
 
 @pytest.mark.parametrize("physics", ["elastic", "acoustic", "sh", "tmem"])
-@pytest.mark.parametrize("axis,cell", [("x", (20, 100)), ("y", (75, 20))])
-def test_resident_infinities_beside_the_frame(physics, axis, cell):
+@pytest.mark.parametrize("rows,axis,cell", [(0, "x", (20, 100)), (0, "y", (75, 20)), (4, "x", (20, 100)),
+                                            (4, "y", (75, 11)), (8, "y", (75, 131))])
+def test_resident_infinities_beside_the_frame(physics, rows, axis, cell):
     """A field that overflows: cells that a CPML frame only shares a tile or a wavefront with have no memory
     variables, so an infinite derivative stays one, as in the two-launch kernels (0 times infinity is NaN)."""
     NX, NY, NT = 150, 140, 20
-    c = _case(physics, NX, NY, NT, 4, 1, 2)
+    c = _case(physics, NX, NY, NT, 4, 1, 2, W=9)
     # a field that is differentiated along the axis, and receivers of what its derivative goes to
     field = {"x": {"elastic": 2, "acoustic": 2, "sh": 1, "tmem": 1},
              "y": {"elastic": 4, "acoustic": 2, "sh": 2, "tmem": 0}}[axis][physics]
@@ -111,6 +131,8 @@ def test_resident_infinities_beside_the_frame(physics, axis, cell):
     seis, fields = [], []
     for kw in (dict(), dict(path=TWO[physics], tile_y=16)):
         s = cases.make_solver(c, **kw)
+        if rows and not kw:
+            s.resident_plan(rows, 8)
         w = s.wavefield(field, 0)
         w[cell[0] + cell[1] * NX] = np.inf
         s.set_wavefield(field, w, 0)

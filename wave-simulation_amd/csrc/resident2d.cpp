@@ -89,8 +89,7 @@ static double two_launch_us(int physics, double cells)
     return 7.0 + cells * (physics == ELASTIC ? 1.3e-5 : 9.1e-6);
 }
 
-// srow != 0: that many rows per wavefront, with the record of the derivative sums
-Res2DPlan res2d_plan(int physics, int order, const Layout2D &L, int nshots, int srow, double *gain)
+Res2DPlan res2d_plan(int physics, int order, const Layout2D &L, int nshots, int srow, int nwv, bool rec, double *gain)
 {
     Res2DPlan best;
     *gain = 0.0;
@@ -104,6 +103,7 @@ Res2DPlan res2d_plan(int physics, int order, const Layout2D &L, int nshots, int 
         if (res_lds(physics, H, S * wmax) + 1024 > 160 * 1024) continue;
         int cap[17] = {};
         for (int w = 1; w <= wmax; w++) {
+            if (nwv && w != nwv) continue;
             Res2DPlan p;
             p.nwv = w;
             p.srow = S;
@@ -115,7 +115,7 @@ Res2DPlan res2d_plan(int physics, int order, const Layout2D &L, int nshots, int 
             p.conc = 1;
             const long long per = (long long)p.nbx * p.nby;
             if (per > 4096) continue;
-            cap[w] = res_capacity(physics, order, p, srow != 0);
+            cap[w] = res_capacity(physics, order, p, rec);
             if (per > cap[w]) continue;
             const int most = cap[w] / (int)per, rounds = (nshots + most - 1) / most;
             p.conc = (nshots + rounds - 1) / rounds;
@@ -162,6 +162,7 @@ struct Res2DState {
     double gain = 0.0;  // estimated step time of the two-launch kernels over that of the plan
     bool planned = false, lists = false;
     int srow = 0;
+    int want_rows = 0, want_waves = 0;  // wv_resident_plan
     std::vector<void *> allocs;      // exchange buffer, control words
     std::vector<void *> acq_allocs;  // lists of the plan's tiles
     int *bsrc_ptr = nullptr, *bsrc = nullptr, *brec_ptr = nullptr, *brec = nullptr;
@@ -310,7 +311,8 @@ static bool res_plan(wv_solver *s, int srow)
     s->free_list(r->acq_allocs);
     s->free_list(r->allocs);
     r->lists = false;
-    r->plan = wv::res2d_plan(s->physics, s->cfg.spatial_fd_order, s->L, s->cfg.nshots, srow, &r->gain);
+    r->plan = wv::res2d_plan(s->physics, s->cfg.spatial_fd_order, s->L, s->cfg.nshots, srow ? srow : r->want_rows,
+                             r->want_waves, srow != 0, &r->gain);
     r->planned = true;
     r->srow = srow;
     r->xch = nullptr;
@@ -333,7 +335,7 @@ size_t res2d_bytes(wv_solver *s, int srow)
 {
     if (!res2d_eligible(s)) return 0;
     double gain = 0.0;
-    const wv::Res2DPlan p = wv::res2d_plan(s->physics, s->cfg.spatial_fd_order, s->L, s->cfg.nshots, srow, &gain);
+    const wv::Res2DPlan p = wv::res2d_plan(s->physics, s->cfg.spatial_fd_order, s->L, s->cfg.nshots, srow, 0, srow != 0, &gain);
     if (!p) return 0;
     int phase1 = 0;
     size_t n = wv::res2d_words(s->physics, s->H, p.rows(), &phase1) * p.blocks() * sizeof(unsigned long long);
@@ -494,7 +496,10 @@ int res2d_run(wv_solver *s, int t0, int nsteps, const wv::Rec2D *rec)
 }
 
 // Whether the planner expects the resident loop to be the faster one for the handle's run calls.
-bool res2d_expected(wv_solver *s, bool rec) { return res_plan(s, rec ? s->tile_y / 4 : 0) && s->res->gain > 1.05; }
+bool res2d_expected(wv_solver *s, bool rec)
+{
+    return res_plan(s, rec ? s->tile_y / 4 : 0) && (s->res->want_rows || s->res->want_waves || s->res->gain > 1.05);
+}
 
 // A wait inside a resident launch ran out: the state is not valid until wv_reset. (Every call that would go
 // on from the state or hand it out asks here first. The report names the launch, so it outlives the buffers
@@ -526,4 +531,31 @@ bool res2d_timed(const wv_solver *s) { return s->res && s->res->timed; }
 void res2d_timing_reset(wv_solver *s)
 {
     if (s->res) s->res->timed = false;
+}
+
+extern "C" int wv_resident_plan(wv_solver *s, int rows, int waves, int *plan)
+{
+    if (!s || !s->inited) return fail(WV_ESTATE, "not initialised");
+    if (!res2d_eligible(s)) return fail(WV_EINVAL, "the resident loop does not take the runs of this handle");
+    if ((rows != 0 && rows != 1 && rows != 2 && rows != 4 && rows != 8) || waves < 0 || waves > 16)
+        return fail(WV_EINVAL, "rows per wavefront must be 0, 1, 2, 4 or 8, wavefronts 0 to 16");
+    if (const int rc = res2d_settle(s); rc < 0) return rc;
+    if (!s->res) s->res = new Res2DState();
+    Res2DState *r = s->res;
+    const int was[2] = {r->want_rows, r->want_waves};
+    r->want_rows = rows;
+    r->want_waves = waves;
+    r->planned = false;
+    if (!res_plan(s, 0)) {
+        r->want_rows = was[0];
+        r->want_waves = was[1];
+        r->planned = false;
+        return fail(WV_EINVAL, "no such plan of the resident loop fits");
+    }
+    if (plan) {
+        plan[0] = r->plan.srow;
+        plan[1] = r->plan.nwv;
+        plan[2] = r->plan.conc;
+    }
+    return WV_OK;
 }

@@ -62,9 +62,10 @@ struct ResGo {
     size_t lds;
 };
 
-// The plan the estimate prefers (empty: none fits); *gain = estimated step time of the two-launch
+// The plan the estimate prefers (empty: none fits) among those with `srow` rows per wavefront and `nwv` wavefronts
+// (0: any), rec: of the kernel that records the derivative sums; *gain = estimated step time of the two-launch
 // kernels over the plan's.
-Res2DPlan res2d_plan(int physics, int order, const Layout2D &L, int nshots, int srow, double *gain);
+Res2DPlan res2d_plan(int physics, int order, const Layout2D &L, int nshots, int srow, int nwv, bool rec, double *gain);
 // exchange words of a block; *phase1: first one of the stress-type phase
 size_t res2d_words(int physics, int H, int rows, int *phase1);
 // Returns the launch status (cooperative launch: every block is resident or nothing runs).

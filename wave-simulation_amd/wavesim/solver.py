@@ -138,6 +138,13 @@ class ForwardSolver:
         self.kernel_choice = self.TUNE_CHOICES[ch.value] if ch.value >= 0 else "plain"
         return self.kernel_choice
 
+    def resident_plan(self, rows=0, waves=0):
+        """Division of the resident 2D loop's work for the following runs (0: the planner's choice); returns
+        (rows per wavefront, wavefronts per block, shots in flight).  The results do not depend on it."""
+        plan = (C.c_int * 3)()
+        _abi.check(_abi.load().wv_resident_plan(self._h, int(rows), int(waves), plan))
+        return tuple(plan)
+
     def synchronize(self):
         _abi.check(_abi.load().wv_synchronize(self._h))
 
