@@ -11,7 +11,9 @@ Printed JSON line: value = grid-cell updates/s of the hand-written kernels
 (kernel variant chosen by the autotuner); `roofline` = algorithmic HBM bytes of
 one time step (60 B per cell-update for 2D elastic plus the CPML memory
 variables of the frame cells) over the GPU time of one time step's kernels
-(start/stop events attached to each dispatch on the solver's stream); the same
+(start/stop events attached to each dispatch on the solver's stream), or, where
+the resident loop runs, which keeps fields and coefficients on the chip, the
+step's arithmetic over that time against the FP32 issue rate; the same
 workload on the reference-sequence GPU path ("plain", one kernel per LAMA
 operation) for the shots/s ratio; `parity`: the GPU seismograms against the
 oracle's float and double runs of the whole shot; and the CPU baseline: the
@@ -31,6 +33,8 @@ for p in (ROOT, os.path.join(ROOT, "wave-simulation_amd")):
         sys.path.insert(0, p)
 
 HBM_PEAK_GBS = 8000.0
+# FP32 operations of 256 CUs x 64 lanes at 2.4 GHz, a multiply-add counted as two (the packed forms are not used)
+FP32_PEAK_GFLOPS = 256 * 64 * 2 * 2.4
 METRIC = "grid-cell updates/s (% HBM peak); batched+adjoint shots/s vs plain at 1e-5"
 
 # Algorithmic HBM bytes of one time step (FP32; every field read and written once, every
@@ -51,6 +55,15 @@ def alg_bytes_per_step(kind, NX, NY, NZ=1, B=1, W=0):
     else:
         frame = 2 * W * (NY + NX)
     return B * cells * 4 * (2 * nf + nc / B) + B * npsi * 8 * frame
+
+
+# Arithmetic of one cell and time step, FP32: derivatives of `order` taps and what is left of the update
+PHYS_FLOPS = {"elastic2d": (8, 20), "tmem": (4, 8)}
+
+
+def alg_flops_per_step(kind, NX, NY, B=1, order=8):
+    nd, rest = PHYS_FLOPS[kind]
+    return float(B) * NX * NY * (2 * order * nd + rest)
 
 
 def parse():
@@ -114,13 +127,23 @@ def _traffic(kernel, path=TRAFFIC_FILE):
     return None
 
 
-def _step_roofline(kernels, steps, alg_bytes, traffic_file=None):
+def _step_roofline(kernels, steps, alg_bytes, traffic_file=None, alg_flops=None):
     """Roofline of one time step: the algorithmic bytes of a step over the GPU time of the step's kernels
     (dispatch-attached events, summed over the kernels of `steps` eager time steps); `traffic` = the HBM bytes
     the step's kernels move, from the committed counter summary of the same workload and kernel variant (null
     when there is none)."""
     run = [k for k in kernels if k["launches"]]
     step_ms = sum(k["avg_ms"] * k["launches"] for k in run) / steps
+    model = [{"name": k["name"], "avg_us": round(k["avg_ms"] * 1e3, 3), "launches": k["launches"],
+              "model_bytes_per_launch": k["bytes"]} for k in run]
+    if any(k["name"] == "res2d" for k in run):
+        # the resident loop keeps fields and coefficients on the chip: its arithmetic against the FP32 issue
+        # rate; `traffic` = halo words, memory variables and samples of a step, which the caches serve
+        achieved = alg_flops / (step_ms * 1e-3) / 1e9
+        return {"bound": "fp32", "achieved": round(achieved, 1), "peak": FP32_PEAK_GFLOPS, "unit": "GFLOP/s",
+                "frac": round(achieved / FP32_PEAK_GFLOPS, 4), "traffic": run[0]["bytes"],
+                "kernel": "res2d (one time step)", "step_us": round(step_ms * 1e3, 3),
+                "alg_flops_per_step": alg_flops, "kernel_model": model}
     achieved = alg_bytes / (step_ms * 1e-3) / 1e9
     main = [k for k in run if k["launches"] >= steps]  # the per-step kernels (not the end-of-run flush)
     traffic = None
@@ -131,8 +154,7 @@ def _step_roofline(kernels, steps, alg_bytes, traffic_file=None):
             "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
             "kernel": " + ".join(k["name"] for k in main) + " (one time step)",
             "step_us": round(step_ms * 1e3, 3), "alg_bytes_per_step": alg_bytes,
-            "kernel_model": [{"name": k["name"], "avg_us": round(k["avg_ms"] * 1e3, 3), "launches": k["launches"],
-                              "model_bytes_per_launch": k["bytes"]} for k in run]}
+            "kernel_model": model}
 
 
 VARIANTS = {"phased-8": ("phased", 8), "phased-16": ("phased", 16), "phased-32": ("phased", 32),
@@ -184,7 +206,8 @@ def bench_batched_tmem(variant="", plain_leg=True):
            "grid_cell_updates_per_s": round(case.cells * NT * n / tb, 1),
            "roofline": _step_roofline(kern, 300, alg_bytes_per_step("tmem", s["NX"], s["NY"], 1, n,
                                                                     s["boundary_width"]),
-                                      TRAFFIC_TMEM if choice == "phased-16" else None)}
+                                      TRAFFIC_TMEM if choice == "phased-16" else None,
+                                      alg_flops_per_step("tmem", s["NX"], s["NY"], n))}
     if plain_leg:
         plain = cases.make_solver(case, path="plain", shots=[case.shots[0]])
         ps = 300
@@ -288,7 +311,8 @@ def bench_batched_elastic(wavesim, L, nshots=8, variant=""):
             "shots_per_s": round(nshots / (ms * 1e-3), 3), "ms_per_step": round(ms / NT, 4),
             "roofline": _step_roofline(kern, 200, alg_bytes_per_step("elastic2d", s["NX"], s["NY"], 1, nshots,
                                                                      s["boundary_width"]),
-                                       TRAFFIC_BATCHED if choice == "strip-16" else None)}
+                                       TRAFFIC_BATCHED if choice == "strip-16" else None,
+                                       alg_flops_per_step("elastic2d", s["NX"], s["NY"], nshots))}
 
 
 def bench_3d(wavesim, L, variant=""):
@@ -481,7 +505,8 @@ def main():
     sol.synchronize()
     kernels = _kernel_stats(sol, L, wavesim)
     wavesim._abi.check(L.wv_set_kernel_timing(sol._h, 0))
-    roofline = _step_roofline(kernels, NT, step_bytes, TRAFFIC_FILE if choice == "strip-16" else None)
+    roofline = _step_roofline(kernels, NT, step_bytes, TRAFFIC_FILE if choice == "strip-16" else None,
+                              alg_flops_per_step("elastic2d", s["NX"], s["NY"]))
 
     out = {
         "metric": METRIC,
@@ -505,7 +530,8 @@ def main():
                    "launches_per_time_step": (0 if choice == "resident" else  # one launch per shot
                                               1 if choice.startswith("fused") else 2),
                    "steps_per_graph": args.graph, "shots_per_step": 1},
-        # the step's algorithmic bytes over the whole timed loop (graphs, flushes, resets included)
+        # the step's algorithmic bytes over the whole timed loop (graphs, flushes, resets included); the
+        # resident loop keeps them on the chip, so for it this compares rates, not HBM use
         "hbm_frac_step": round(step_bytes * NT * args.steps / wall / 1e9 / HBM_PEAK_GBS, 4),
         "gpu_event_ms_per_step": round(gpu_ms / args.steps, 3),
         "roofline": roofline,

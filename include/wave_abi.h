@@ -194,8 +194,9 @@ int wv_last_run_ms(wv_solver *s, double *ms);
  * the kernel name, its average duration [ms] per launch, the number of
  * launches, and the algorithmic HBM bytes one launch must move (every field
  * and coefficient of the batch read once, updated fields written once, CPML
- * memory variables read and written on frame cells).  Returns WV_EINVAL for an
- * unknown kind.  No counterpart in the reference (instrumentation only). */
+ * memory variables read and written on frame cells).  The resident loop is reported as kind 0,
+ * counted per time step, with the bytes a step moves outside the compute units (halo words, CPML memory
+ * variables or ABS factors, samples).  Returns WV_EINVAL for an unknown kind.  No counterpart in the reference (instrumentation only). */
 int wv_set_kernel_timing(wv_solver *s, int on);
 int wv_kernel_stats(wv_solver *s, int kind, const char **name, double *avg_ms, long long *launches,
                     double *bytes_per_launch);

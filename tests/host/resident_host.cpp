@@ -422,6 +422,27 @@ void plan()
     CHECK(wv_resident_plan(&s, 0, 0, p) == WV_EINVAL);
 }
 
+// The bytes reported for a step: every tile sends H rows or columns of its border, two fields per phase, to
+// each neighbour, and every cell of the frames moves four memory variables.
+void step_bytes()
+{
+    wv_solver s;
+    make(s);
+    int p[3];
+    CHECK(wv_resident_plan(&s, 4, 8, p) == WV_OK);
+    const int R = 32, nbx = 4, nby = 5, H = 4, W = s.cfg.boundary_width = 10;
+    double words = 0, psi = 0;
+    for (int by = 0; by < nby; by++)
+        for (int bx = 0; bx < nbx; bx++) {
+            const int rows = std::min(R, 150 - by * R), columns = std::min(64, 200 - bx * 64);
+            words += 2 * 2 * H * (((bx > 0) + (bx + 1 < nbx)) * rows + ((by > 0) + (by + 1 < nby)) * columns);
+        }
+    for (int y = 0; y < 150; y++)
+        for (int x = 0; x < 200; x++) psi += 4 * (wv::frame_index(x, 200, W, false) >= 0) + 4 * (wv::frame_index(y, 150, W, false) >= 0);
+    const double samples = 2;  // one source per shot; no receivers are set up here
+    CHECK(res2d_step_bytes(&s) == 2 * (words * 8 * 2 + psi * 4 * 2) + samples * 4);
+}
+
 // Read-backs take what device memory there is, down to one item, then pinned host memory.
 void staging()
 {
@@ -478,6 +499,8 @@ int main(int argc, char **argv)
         queue();
     else if (t == "plan")
         plan();
+    else if (t == "step_bytes")
+        step_bytes();
     else if (t == "staging")
         staging();
     else

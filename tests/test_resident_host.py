@@ -18,7 +18,8 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("test", ["no_memory", "memory_asked_for", "timing", "failure", "refusal", "queue", "plan", "staging"])
+@pytest.mark.parametrize("test", ["no_memory", "memory_asked_for", "timing", "failure", "refusal", "queue", "plan",
+                                  "step_bytes", "staging"])
 def test_resident_host(program, test):
     r = subprocess.run([program, test], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout.strip() == "ok", r.stderr

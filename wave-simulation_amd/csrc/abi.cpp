@@ -1378,7 +1378,7 @@ int wv_kernel_stats(wv_solver *s, int kind, const char **name, double *avg_ms, l
     if (avg_ms) *avg_ms = s->klaunch[kind] ? s->kms[kind] / s->klaunch[kind] : 0.0;
     if (bytes_per_launch)
         *bytes_per_launch = !res2d_timed(s) || kind > 1 ? s->kernel_bytes(kind)
-                            : (kind == 0 ? s->kernel_bytes(0) + s->kernel_bytes(1) : 0.0);
+                            : (kind == 0 ? res2d_step_bytes(s) : 0.0);
     return WV_OK;
 }
 

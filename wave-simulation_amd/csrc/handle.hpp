@@ -324,4 +324,5 @@ bool res2d_failed(const wv_solver *s);
 int res2d_reset(wv_solver *s);
 extern const char *const kResidentFailed;
 bool res2d_timed(const wv_solver *s);  // the timed run calls went through the resident loop
+double res2d_step_bytes(const wv_solver *s);
 void res2d_timing_reset(wv_solver *s);

@@ -71,8 +71,9 @@ static int res_capacity(int physics, int order, const Res2DPlan &p, bool rec)
 
 // Estimated us per time step of the whole batch: rounds x (exchange, barriers and latency of a step +
 // the arithmetic of the rows a CU holds).  Measured (MI355X, order 8; us per round): elastic 64 rows
-// per CU 11.9 (one block of 16 x 4 rows) and 12.4 (two of 8 x 4), 16 rows 5.7; TM-EM 64 rows 6.4 - 6.7;
-// SH 64 rows 6.0, 128 rows 10.4; acoustic order 4: 4 rows 3.5, 64 rows 4.7.
+// per CU 11.9 (one block of 16 x 4 rows; 10.9 since, which leaves the choices as they are) and 12.4 (two of
+// 8 x 4), 16 rows 5.7; TM-EM 64 rows 6.4 - 6.7; SH 64 rows 6.0, 128 rows 10.4; acoustic order 4: 4 rows 3.5,
+// 64 rows 4.7.
 static double res_step_us(int physics, int order, const Res2DPlan &p, int nshots)
 {
     const int rounds = (nshots + p.conc - 1) / p.conc, cus = std::max(1, wv_cu_count());
@@ -525,6 +526,23 @@ int res2d_reset(wv_solver *s)
     if (r->refused < 3) r->off = false;
     if (r->xch) HIP_TRY(hipMemsetAsync(r->ctl + 2, 0, 2 * sizeof(unsigned), s->st));
     return 0;
+}
+
+// Bytes that a step of the whole batch moves outside the CUs: halo words (8 bytes, written and read, H deep on
+// both sides of every edge between tiles), CPML memory variables (read and written), ABS factors, samples.
+// The load and the store of the state at the ends of a run call are not in it.
+double res2d_step_bytes(const wv_solver *s)
+{
+    if (!s->res || !s->res->plan) return 0.0;
+    const wv::Res2DPlan &p = s->res->plan;
+    const double B = s->cfg.nshots, nf = s->physics == wv::ELASTIC ? 2 : 1, W = s->cfg.boundary_width;
+    double bytes = B * 2 * 8 * 2 * nf * 2 * s->H * ((p.nbx - 1.0) * s->cfg.NY + (p.nby - 1.0) * s->cfg.NX);
+    if (s->cfg.damping_boundary == 2)
+        bytes += B * 8 * 2 * nf * (2 * W * s->cfg.NY + (s->cfg.free_surface ? W : 2 * W) * s->cfg.NX);
+    if (s->cfg.damping_boundary == 1) bytes += B * 4 * (double)s->cfg.NX * s->cfg.NY;
+    double samples = s->rec_total;
+    for (const ShotAcq &a : s->shots) samples += a.sidx.size();
+    return bytes + 4 * samples;
 }
 
 bool res2d_timed(const wv_solver *s) { return s->res && s->res->timed; }
