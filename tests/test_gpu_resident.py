@@ -8,11 +8,13 @@ many rows, every order, CPML / ABS / rigid edges with and without a free surface
 a wavefront and more receivers than a block holds, several rounds of shots, runs cut into pieces,
 queued runs, and the adjoint's record.
 """
+import ctypes as C
 import time
 
 import numpy as np
 import pytest
 
+import wavesim
 from wavesim import cases
 
 pytestmark = pytest.mark.gpu
@@ -74,6 +76,29 @@ def test_resident_rows_per_wavefront(physics, rows, order, tile, damping, fs):
     NY = max(3 * order, 2 * R + R // 2 + 3, 45)
     c = _case(physics, 150, NY, 150, order, 2, damping, fs=fs if physics != "tmem" else 0, W=10)
     _equal(c, 150, pieces=[25], plan=(rows, waves))
+
+
+@pytest.mark.parametrize("physics", ["elastic", "acoustic", "sh", "tmem"])
+@pytest.mark.parametrize("order", [2, 4, 6, 8, 10, 12])
+def test_resident_plans_fit_the_device(physics, order):
+    """The planner counts no more blocks than are resident at once: with shots enough for the whole chip, every
+    division of the work runs in the loop, and none is refused at its check-in."""
+    c = _case(physics, 70, 45, 16, order, 1, 0)
+    c.shots = c.shots * 700
+    s = cases.make_solver(c)
+    L = wavesim.load()
+    wavesim._abi.check(L.wv_set_kernel_timing(s._h, 1))
+    for rows in (1, 2, 4, 8):
+        for waves in range(1, 17):
+            try:
+                plan = s.resident_plan(rows, waves)
+            except wavesim.WaveError:
+                continue
+            wavesim._abi.check(L.wv_set_kernel_timing(s._h, 1))
+            s.run(0, 16)
+            name, n = C.c_char_p(), C.c_longlong()
+            wavesim._abi.check(L.wv_kernel_stats(s._h, 0, C.byref(name), None, C.byref(n), None))
+            assert name.value == b"res2d" and n.value == 16, plan
 
 
 @pytest.mark.parametrize("physics", ["elastic", "acoustic"])

@@ -66,7 +66,13 @@ static int res_capacity(int physics, int order, const Res2DPlan &p, bool rec)
     }
     // a block whose wavefronts do not spread evenly over the four SIMDs of a CU may find no place beside
     // another one although registers and LDS would do in sum: count one block per CU then
-    return p.nwv % 4 ? std::min(cap, wv_cu_count()) : cap;
+    const int cus = wv_cu_count();
+    if (p.nwv % 4) cap = std::min(cap, cus);
+    // Two things the estimate does not know. A block is given LDS in units of 1280 bytes (five blocks of
+    // 32,440 bytes do not fit 160 KB); and a SIMD takes six wavefronts of these kernels, whose scalar
+    // registers are all in use, where it says seven (1792 blocks of four wavefronts, 1536 come in).
+    const size_t lds = (g.lds + 16 + 1279) / 1280 * 1280;
+    return std::min(cap, cus * std::min((int)(160 * 1024 / lds), std::max(1, 6 / ((p.nwv + 3) / 4))));
 }
 
 // Estimated us per time step of the whole batch: rounds x (exchange, barriers and latency of a step +
