@@ -183,11 +183,14 @@ __device__ __forceinline__ res_args fresh_args(res_args p)
 }
 #define RES_GLOBAL __attribute__((address_space(1)))
 
-// a of the rows outside the y frame that share a wavefront with rows of it.  Their psi is this times the
-// derivative (and zero again when the next step loads it): added to the derivative, it changes no finite
-// one, being far below half a unit in the last place, and leaves an infinite one as it is, which the
-// tables' 0 would make NaN.  A select on each result instead: 11.8 -> 12.1 us per step of 1000 x 1000
-// elastic cells; zeroing what is stored, as here: 11.5 -> 11.0.
+// Cells outside a CPML frame that share a tile or a wavefront with it have a = b = 0 in the tables, which
+// leaves a finite derivative as it is but makes an infinite one NaN.  Lanes outside the x frame take no
+// part in its update (where the registers are full, 8 rows of three fields, a select on psi costs less: SELX).
+// Rows outside the y frame: a select on psi with three fields; with the five of P-SV an a that changes no
+// finite derivative, psi being far below half a unit in its last place, and leaves an infinite one as
+// it is, with zeros stored for psi (SELY).  us per step, with selects for x and y and without: 1000 x 1000
+// elastic 12.1 and 10.9; 428 x 392 TM-EM of 40 shots at order 10 (8 rows) 59.9 and 61.5, 882 x 482 of 5 at
+// order 4 (4 rows) 13.7 and 13.6.
 constexpr float RES_OUTSIDE_A = 1e-30f;
 
 // Floats of a wavefront's private memory variables: two phases x (x frame, y frame) x NP * S rows.
@@ -206,6 +209,7 @@ __global__ __launch_bounds__(MAXT, MINW) void res2d(Res2DKernArgs KA)
     constexpr int NF = RF::NF, K = 2 * H + 1, RW = TILE_X + 2 * H, NW = S + 2 * H;
     constexpr int RMAX = MAXT / 64 * S, FS = (RMAX + 2 * H) * RW;  // LDS strides of the largest tile: constants
     constexpr int NP = PHYS == ELASTIC ? 2 : 1;   // memory variables per phase and axis
+    constexpr bool SELY = PHYS != ELASTIC, SELX = SELY && S == 8;  // see RES_OUTSIDE_A
     constexpr int PV = NP * S >= 4 ? 4 : NP * S;  // floats per access of the private memory variables
     typedef float vpsi __attribute__((ext_vector_type(PV)));
     extern __shared__ float lds[];
@@ -246,7 +250,7 @@ __global__ __launch_bounds__(MAXT, MINW) void res2d(Res2DKernArgs KA)
 #pragma unroll
         for (int h = 0; h < 2; h++) {
             const float a = on ? (h ? KA.P.ayh : KA.P.ay)[y0 + e] : 0.f, b = on ? (h ? KA.P.byh : KA.P.by)[y0 + e] : 0.f;
-            s_cy[4 * e + 2 * h] = a != 0.f || b != 0.f ? a : RES_OUTSIDE_A;
+            s_cy[4 * e + 2 * h] = SELY || a != 0.f || b != 0.f ? a : RES_OUTSIDE_A;
             s_cy[4 * e + 2 * h + 1] = b;
         }
     }
@@ -378,7 +382,7 @@ __global__ __launch_bounds__(MAXT, MINW) void res2d(Res2DKernArgs KA)
         if (tid < nr) rid = receiver(G0, tid, ro1, ro2);
         // memory variables (stress phase under ABS: the damping factors, in px) of the next phase,
         // loaded before the wait for its halos
-        // (rows outside the y frame store zeros, so they load zeros every time)
+        // (rows outside the y frame store zeros, and load zeros every time)
         float px[NP * S], py[NP * S];
 #pragma unroll
         for (int k = 0; k < NP * S; k++) px[k] = py[k] = 0.f;
@@ -399,25 +403,39 @@ __global__ __launch_bounds__(MAXT, MINW) void res2d(Res2DKernArgs KA)
             const res_args G = fresh_args(G0);
             if (xf) psi_store(G, ph, 0, px);
             if (yframe) {
-                if constexpr (S > 1) {
+                if constexpr (S > 1 && !SELY) {
 #pragma unroll
-                for (int k = 0; k < NP * S; k++) py[k] = yrows >> k % S & 1 ? py[k] : 0.f;
+                    for (int k = 0; k < NP * S; k++) py[k] = yrows >> k % S & 1 ? py[k] : 0.f;
                 }
                 psi_store(G, ph, 1, py);
             }
         };
-        // CPML of the derivative d of every row: memory variable j of a phase, profile full or half (x: in the
-        // lanes of the frame; y: rows outside the frame have RES_OUTSIDE_A)
+        // CPML of the derivative d of every row: memory variable j of a phase, profile full or half
+        // (outside the frames: see RES_OUTSIDE_A)
         auto cpml_x = [&](int j, float (&d)[S], bool half) {
             const float a = half ? col.axh : col.ax, b = half ? col.bxh : col.bx;
 #pragma unroll
-            for (int r = 0; r < S; r++) px[j * S + r] = cpml(d[r], px[j * S + r], a, b);
+            for (int r = 0; r < S; r++) {
+                if constexpr (SELX) {
+                    const float p = __builtin_fmaf(a, d[r], b * px[j * S + r]);
+                    px[j * S + r] = xf ? p : 0.f;
+                    d[r] += px[j * S + r];
+                } else {
+                    px[j * S + r] = cpml(d[r], px[j * S + r], a, b);
+                }
+            }
         };
         auto cpml_y = [&](int j, float (&d)[S], bool half, int row) {
 #pragma unroll
             for (int r = 0; r < S; r++) {
                 const float *cy = s_cy + 4 * (row + r) + (half ? 2 : 0);
-                py[j * S + r] = cpml(d[r], py[j * S + r], cy[0], cy[1]);
+                if constexpr (S > 1 && SELY) {
+                    const float p = __builtin_fmaf(cy[0], d[r], cy[1] * py[j * S + r]);
+                    py[j * S + r] = yrows >> r & 1 ? p : 0.f;
+                    d[r] += py[j * S + r];
+                } else {
+                    py[j * S + r] = cpml(d[r], py[j * S + r], cy[0], cy[1]);
+                }
             }
         };
         // y derivative of field f at the wavefront's rows from a column window in registers; INNER: the
@@ -526,7 +544,7 @@ __global__ __launch_bounds__(MAXT, MINW) void res2d(Res2DKernArgs KA)
                 y_rows(inner_c, PHYS == TMEM ? G->T.yf : G->T.yf_v, G->T.yf, 2, lr0, ya, v);
                 x_rows(cxf, 2, lr0, u);
             }
-            if (xf) {
+            if (SELX ? xframe : xf) {
                 cpml_x(0, u, PHYS != SH);
                 if constexpr (PHYS == ELASTIC) cpml_x(1, a, false);
             }
@@ -583,7 +601,7 @@ __global__ __launch_bounds__(MAXT, MINW) void res2d(Res2DKernArgs KA)
                 y_rows(inner_c, G->T.yb, G->T.yb, PHYS == ACOUSTIC ? 1 : 0, lr0, ya, v);
                 x_rows(cxb, PHYS == ACOUSTIC ? 0 : 1, lr0, u);
             }
-            if (xf) {
+            if (SELX ? xframe : xf) {
                 cpml_x(0, u, PHYS == SH);
                 if constexpr (PHYS == ELASTIC) cpml_x(1, a, true);
             }
