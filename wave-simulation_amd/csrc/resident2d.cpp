@@ -314,7 +314,10 @@ static bool res_plan(wv_solver *s, int srow)
     if (r->planned && r->srow == srow) return (bool)r->plan;
     // the queued launches use the buffers of the plan that goes (refused ones: the caller finds the loop
     // off, and settles before it runs anything)
-    if (!r->queued.empty() && (hipStreamSynchronize(s->st) != hipSuccess || res_verdicts(r) != 1)) return false;
+    {
+        std::lock_guard<std::mutex> hold(r->lock);
+        if (!r->queued.empty() && (hipStreamSynchronize(s->st) != hipSuccess || res_verdicts(r) != 1)) return false;
+    }
     s->free_list(r->acq_allocs);
     s->free_list(r->allocs);
     r->lists = false;
